@@ -43,9 +43,12 @@ __global__ void k_bs0(int n, const double *a, double *b) {
 }
 
 // ---------------------------------------------------------------------- BS1 --
+// n / 2 pairs, and the last entry of an odd n (a launch of its own for that
+// entry: axpy of 10007 entries 6.9 us per call against 3.8)
 template <int U, bool NT>
-__global__ __launch_bounds__(256) void k_copy2(int64_t n2, const dbl2 *__restrict__ a,
+__global__ __launch_bounds__(256) void k_copy2(int64_t n, const dbl2 *__restrict__ a,
                                                dbl2 *__restrict__ b) {
+  const int64_t n2 = n / 2;
   const int64_t base = (int64_t)blockIdx.x * (U * 256) + threadIdx.x;
   dbl2 r[U];
 #pragma unroll
@@ -58,20 +61,23 @@ __global__ __launch_bounds__(256) void k_copy2(int64_t n2, const dbl2 *__restric
     const int64_t i = base + u * 256;
     if (i < n2) st2<NT>(b + i, r[u]);
   }
+  if ((n & 1) && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+    reinterpret_cast<double *>(b)[n - 1] = reinterpret_cast<const double *>(a)[n - 1];
 }
 
-// scalar path for unaligned pointers and the odd tail element
-__global__ __launch_bounds__(256) void k_copy1(int64_t lo, int64_t n, const double *__restrict__ a,
+// scalar path for unaligned pointers
+__global__ __launch_bounds__(256) void k_copy1(int64_t n, const double *__restrict__ a,
                                                double *__restrict__ b) {
-  int64_t i = lo + (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * 256;
   for (; i < n; i += st) b[i] = a[i];
 }
 
 // ---------------------------------------------------------------------- BS2 --
 template <int U, bool NT>
-__global__ __launch_bounds__(256) void k_axpy2(int64_t n2, double alpha, const dbl2 *__restrict__ x,
+__global__ __launch_bounds__(256) void k_axpy2(int64_t n, double alpha, const dbl2 *__restrict__ x,
                                                double beta, dbl2 *__restrict__ y) {
+  const int64_t n2 = n / 2;
   const int64_t base = (int64_t)blockIdx.x * (U * 256) + threadIdx.x;
   dbl2 rx[U], ry[U];
 #pragma unroll
@@ -92,12 +98,16 @@ __global__ __launch_bounds__(256) void k_axpy2(int64_t n2, double alpha, const d
       st2<NT>(y + i, o);
     }
   }
+  if ((n & 1) && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    double *yl = reinterpret_cast<double *>(y) + (n - 1);
+    *yl = alpha * reinterpret_cast<const double *>(x)[n - 1] + beta * *yl;
+  }
 }
 
-__global__ __launch_bounds__(256) void k_axpy1(int64_t lo, int64_t n, double alpha,
+__global__ __launch_bounds__(256) void k_axpy1(int64_t n, double alpha,
                                                const double *__restrict__ x, double beta,
                                                double *__restrict__ y) {
-  int64_t i = lo + (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * 256;
   for (; i < n; i += st) y[i] = alpha * x[i] + beta * y[i];
 }
@@ -195,13 +205,20 @@ template <> struct LaneSum<true> {
   __device__ __forceinline__ double value() const { return s + c; }
 };
 
-template <int KIND, int U, bool NT, typename ACC>
-__device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t stride, ACC &acc) {
+// one running sum for the group, or one per entry
+template <bool C> __device__ __forceinline__ LaneSum<C> &lane_of(LaneSum<C> &a, int) { return a; }
+template <bool C, int N> __device__ __forceinline__ LaneSum<C> &lane_of(LaneSum<C> (&a)[N], int u) { return a[u]; }
+
+// LAST: the group may reach past n; entries there are neither loaded, stored
+// nor added.
+template <int KIND, int U, bool NT, bool LAST = false, typename ACC>
+__device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t stride, ACC &acc, int64_t n = 0) {
   double va[U], vb[U], vr[U], vx[U];
   int64_t ix[KIND == RED_CGFULL ? U : 1];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t i = id + u * stride;
+    if (LAST && i >= n) break;
     if constexpr (KIND == RED_CGFULL) {
       ix[u] = x_index(A, i);
       va[u] = ldv<NT>(A.a + ix[u]);
@@ -215,6 +232,7 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t i = id + u * stride;
+    if (LAST && i >= n) break;
     double term;
     if constexpr (KIND == RED_NORM) {
       term = va[u] * va[u];
@@ -230,14 +248,21 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
       stv<NT>(A.r + i, rr);
       term = rr * rr;
     }
-    acc.add(term);
+    lane_of(acc, u).add(term);
   }
 }
 
 // COMP = false: the reference order exactly.  COMP = true (FAST mode): the
 // same launch shape and element order with compensated lane sums, so it runs
 // at the reference order's bandwidth and is more accurate.
-template <int KIND, int BS, int U, bool NT, bool COMP = false>
+// TAIL: the entries past a lane's last whole group of U also go out in groups
+// instead of one memory latency each.  That is taken while a lane has fewer
+// than kTailGroups whole groups (n < 2^25 at 256 x 256 lanes); measured on
+// MI355X, full form, us per call, one by one / in groups: n = 500001 8.6 / 7.3,
+// 900000 11.4 / 10.9, 2000001 23.1 / 20.1, 3000003 31.8 / 28.7, 10000001 89.4 /
+// 87.2, but 2^27 1094 / 1105 (norm, dot and update there within 0.3 %).
+constexpr int kTailGroups = 32;
+template <int KIND, int BS, int U, bool NT, bool COMP, bool TAIL>
 __global__ __launch_bounds__(BS) void k_red_ref1(int64_t n, int64_t nblock, RedArgs A,
                                                  double *__restrict__ partials) {
   __shared__ double s[BS];
@@ -247,7 +272,19 @@ __global__ __launch_bounds__(BS) void k_red_ref1(int64_t n, int64_t nblock, RedA
   LaneSum<COMP> acc;
   for (; id + (int64_t)(U - 1) * stride < n; id += (int64_t)U * stride)
     ref_group<KIND, U, NT>(A, id, stride, acc);
-  for (; id < n; id += stride) acc.add(red_term<KIND>(A, id));
+  if constexpr (TAIL) {
+    // up to U - 1 entries are left: groups of 8 and 4, then one that may reach past n
+    if constexpr (U >= 16) {
+      if (id + 7 * stride < n) {
+        ref_group<KIND, 8, NT>(A, id, stride, acc);
+        id += 8 * stride;
+      }
+    }
+    for (; id + 3 * stride < n; id += 4 * stride) ref_group<KIND, 4, NT>(A, id, stride, acc);
+    if (id < n) ref_group<KIND, 4, NT, true>(A, id, stride, acc, n);
+  } else {
+    for (; id < n; id += stride) acc.add(red_term<KIND>(A, id));
+  }
   s[t] = acc.value();
   __syncthreads();
   const double blk = ref_tree<BS>(s);
@@ -268,6 +305,67 @@ __global__ __launch_bounds__(BS) void k_red_ref2(int64_t nblock, const double *_
   if (t == 0) out[0] = v;
 }
 
+
+// Both stages in one workgroup, for 256-entry blocks with n <= small_n(KIND): each
+// lane of the two-launch form then has one entry, so a wave takes whole
+// blocks, 4 entries of each per lane, and the tree's steps are register adds (128, 64)
+// and lane shifts (32 .. 2, s[0]+s[1]) in the same order; the partials stay in
+// LDS and wave 0 folds them by stage 2's own order.  The result is bit
+// for bit that of the two launches.  Vectors this short cost their launches
+// and one memory latency, not bytes.
+constexpr int kSmallWaves = 16;
+template <bool FAST> __device__ __forceinline__ double small_stage2(const double *part, int nb, int l) {
+  if constexpr (FAST) {  // k_red_fast2, block_sum256
+    double ws[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double s = 0.0, c = 0.0;
+      if (l + 64 * k < nb) neumaier(s, c, part[l + 64 * k]);
+      ws[k] = s + c;
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) ws[k] += __shfl_xor(ws[k], off, 64);
+    }
+    return (ws[0] + ws[1]) + (ws[2] + ws[3]);
+  } else {  // k_red_ref2<256>
+    double e[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      e[k] = 0.0;
+      if (l + 64 * k < nb) e[k] += part[l + 64 * k];
+    }
+    double v = (e[0] + e[2]) + (e[1] + e[3]);
+#pragma unroll
+    for (int w = 32; w >= 1; w >>= 1) v += __shfl_down(v, w, 64);
+    return v;
+  }
+}
+
+template <int KIND, bool COMP>
+__global__ __launch_bounds__(64 * kSmallWaves) void k_red_small(int64_t n, int nb, RedArgs A,
+                                                                double *__restrict__ out) {
+  __shared__ double part[256];
+  constexpr int G = KIND == RED_CGFULL ? 2 : 4;  // blocks of a wave whose loads are in flight together
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int b = wv * G; b < nb; b += kSmallWaves * G) {
+    LaneSum<COMP> acc[4 * G];
+    const int64_t i0 = (int64_t)b * 256;
+    if (i0 + 256 * G <= n) ref_group<KIND, 4 * G, false>(A, i0 + l, 64, acc);
+    else ref_group<KIND, 4 * G, false, true>(A, i0 + l, 64, acc, n);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const LaneSum<COMP> *e = acc + 4 * g;
+      double v = (e[0].value() + e[2].value()) + (e[1].value() + e[3].value());
+#pragma unroll
+      for (int w = 32; w >= 1; w >>= 1) v += __shfl_down(v, w, 64);
+      if (l == 0 && b + g < nb) part[b + g] = v;
+    }
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const double v = small_stage2<COMP>(part, nb, l);
+    if (l == 0) out[0] = v;
+  }
+}
 
 // Block sum of (s + c) over 256 threads with a fixed shape: wave-level
 // shuffles then LDS across the 4 waves.
@@ -312,14 +410,14 @@ static spx_tuning_t stream_defaults() {
 }
 
 template <int U, bool NT>
-static void launch_copy2(unsigned grid, int64_t n2, const double *a, double *b) {
-  hipLaunchKernelGGL((k_copy2<U, NT>), dim3(grid), dim3(256), 0, current_stream(), n2,
+static void launch_copy2(unsigned grid, int64_t n, const double *a, double *b) {
+  hipLaunchKernelGGL((k_copy2<U, NT>), dim3(grid), dim3(256), 0, current_stream(), n,
                      reinterpret_cast<const dbl2 *>(a), reinterpret_cast<dbl2 *>(b));
 }
 template <int U, bool NT>
-static void launch_axpy2(unsigned grid, int64_t n2, double alpha, const double *x, double beta,
+static void launch_axpy2(unsigned grid, int64_t n, double alpha, const double *x, double beta,
                          double *y) {
-  hipLaunchKernelGGL((k_axpy2<U, NT>), dim3(grid), dim3(256), 0, current_stream(), n2, alpha,
+  hipLaunchKernelGGL((k_axpy2<U, NT>), dim3(grid), dim3(256), 0, current_stream(), n, alpha,
                      reinterpret_cast<const dbl2 *>(x), beta, reinterpret_cast<dbl2 *>(y));
 }
 
@@ -338,17 +436,20 @@ static int fast_grid() {
   return g < 1 ? 1 : (g > kFastGridMax ? kFastGridMax : g);
 }
 
-template <int KIND, int BS, bool NT, bool COMP>
-static void launch_ref1_nt(int64_t n, int64_t nb, const RedArgs &A, double *tmp, int unroll) {
-  if (unroll >= 32)
-    hipLaunchKernelGGL((k_red_ref1<KIND, BS, 32, NT, COMP>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
-                       nb, A, tmp);
-  else if (unroll >= 16)
-    hipLaunchKernelGGL((k_red_ref1<KIND, BS, 16, NT, COMP>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
+template <int KIND, int BS, int U, bool NT, bool COMP>
+static void launch_ref1_u(int64_t n, int64_t nb, const RedArgs &A, double *tmp) {
+  if (n < (int64_t)kTailGroups * U * BS * nb)
+    hipLaunchKernelGGL((k_red_ref1<KIND, BS, U, NT, COMP, true>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
                        nb, A, tmp);
   else
-    hipLaunchKernelGGL((k_red_ref1<KIND, BS, 8, NT, COMP>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
+    hipLaunchKernelGGL((k_red_ref1<KIND, BS, U, NT, COMP, false>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
                        nb, A, tmp);
+}
+template <int KIND, int BS, bool NT, bool COMP>
+static void launch_ref1_nt(int64_t n, int64_t nb, const RedArgs &A, double *tmp, int unroll) {
+  if (unroll >= 32) launch_ref1_u<KIND, BS, 32, NT, COMP>(n, nb, A, tmp);
+  else if (unroll >= 16) launch_ref1_u<KIND, BS, 16, NT, COMP>(n, nb, A, tmp);
+  else launch_ref1_u<KIND, BS, 8, NT, COMP>(n, nb, A, tmp);
 }
 template <int KIND, int BS, bool COMP = false>
 static void launch_ref1(int64_t n, int64_t nb, const RedArgs &A, double *tmp, int unroll, bool nt) {
@@ -371,6 +472,14 @@ static spx_tuning_t reference_tuning(int kind) {
   return tuning_for("reduce_reference", d);
 }
 
+// Largest n of the one-launch form (at most 256 * 256).  One workgroup's
+// loads and stores run through one CU, so the line lies where that costs as
+// much as the second launch.  Measured on MI355X, us per call back to back,
+// two launches / one: norm n = 2500 6.3 / 3.7, 16384 6.6 / 4.6; dot 2500 6.5 /
+// 3.9, 16384 6.8 / 6.2; update 5000 6.6 / 5.1, 10007 6.9 / 6.6, 16000 6.9 /
+// 8.3; full form 2500 6.8 / 4.6, 5000 7.0 / 5.9, 10007 6.8 / 8.7.
+constexpr int64_t small_n(int kind) { return kind == RED_CGFULL ? 5120 : kind == RED_CG ? 8192 : 16384; }
+
 template <int KIND>
 static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *tmp, double *out,
                          int mode, int bs) {
@@ -382,6 +491,12 @@ static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *
       return fail(SPX_ERR_ARG, std::string(name) + ": block_size must be 256, 512 or 1024");
     int64_t nb = (n + bs - 1) / bs;
     if (nb > bs) nb = bs;
+    if (bs == 256 && n <= small_n(KIND)) {
+      hipLaunchKernelGGL((k_red_small<KIND, false>), dim3(1), dim3(64 * kSmallWaves), 0, current_stream(), n, (int)nb,
+                         A, out);
+      SPX_LAUNCHED(name);
+      return SPX_OK;
+    }
     const spx_tuning_t t = reference_tuning(KIND);
     const int U = t.unroll > 0 ? t.unroll : 16;
     const bool nt = t.nontemporal > 0;
@@ -403,7 +518,14 @@ static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *
   // element order, compensated lane sums, then a compensated fold of the
   // partials; deterministic for a given grid.
   int64_t nb = (n + 255) / 256;
-  if (nb > fast_grid()) nb = fast_grid();
+  const int64_t grid = fast_grid();
+  if (n <= small_n(KIND) && nb <= grid && nb <= 256) {
+    hipLaunchKernelGGL((k_red_small<KIND, true>), dim3(1), dim3(64 * kSmallWaves), 0, current_stream(), n, (int)nb, A,
+                       out);
+    SPX_LAUNCHED(name);
+    return SPX_OK;
+  }
+  if (nb > grid) nb = grid;
   spx_tuning_t fd = reference_tuning(KIND);  // loads per lane and streaming accesses as the reference order's
   fd.grid_blocks = 0;
   const spx_tuning_t ft = tuning_for("reduce_fast", fd);
@@ -503,23 +625,17 @@ int spx_bs1_copy(int64_t n, const double *a, double *b) {
     const int64_t n2 = n / 2;
     const int U = t.unroll;
     const bool nt = t.nontemporal > 0;
-    if (n2 > 0) {
-      unsigned grid;
-      int rc = vec_blocks(n2, (U >= 8 ? 8 : U >= 4 ? 4 : 2) * 256, &grid);
-      if (rc) return rc;
-      if (U >= 8) nt ? launch_copy2<8, true>(grid, n2, a, b) : launch_copy2<8, false>(grid, n2, a, b);
-      else if (U >= 4) nt ? launch_copy2<4, true>(grid, n2, a, b) : launch_copy2<4, false>(grid, n2, a, b);
-      else nt ? launch_copy2<2, true>(grid, n2, a, b) : launch_copy2<2, false>(grid, n2, a, b);
-      SPX_LAUNCHED("spx_bs1_copy");
-    }
-    if (n & 1) {
-      hipLaunchKernelGGL(k_copy1, dim3(1), dim3(256), 0, current_stream(), n - 1, n, a, b);
-      SPX_LAUNCHED("spx_bs1_copy tail");
-    }
+    unsigned grid;  // at least one block
+    int rc = vec_blocks(n2, (U >= 8 ? 8 : U >= 4 ? 4 : 2) * 256, &grid);
+    if (rc) return rc;
+    if (U >= 8) nt ? launch_copy2<8, true>(grid, n, a, b) : launch_copy2<8, false>(grid, n, a, b);
+    else if (U >= 4) nt ? launch_copy2<4, true>(grid, n, a, b) : launch_copy2<4, false>(grid, n, a, b);
+    else nt ? launch_copy2<2, true>(grid, n, a, b) : launch_copy2<2, false>(grid, n, a, b);
+    SPX_LAUNCHED("spx_bs1_copy");
   } else {
     int64_t g = (n + 255) / 256;
     if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(k_copy1, dim3((unsigned)g), dim3(256), 0, current_stream(), (int64_t)0, n, a, b);
+    hipLaunchKernelGGL(k_copy1, dim3((unsigned)g), dim3(256), 0, current_stream(), n, a, b);
     SPX_LAUNCHED("spx_bs1_copy");
   }
   return SPX_OK;
@@ -535,23 +651,17 @@ int spx_bs2_axpy(int64_t n, double alpha, const double *x, double beta, double *
     const int64_t n2 = n / 2;
     const int U = t.unroll;
     const bool nt = t.nontemporal > 0;
-    if (n2 > 0) {
-      unsigned grid;
-      int rc = vec_blocks(n2, (U >= 8 ? 8 : U >= 4 ? 4 : 2) * 256, &grid);
-      if (rc) return rc;
-      if (U >= 8) nt ? launch_axpy2<8, true>(grid, n2, alpha, x, beta, y) : launch_axpy2<8, false>(grid, n2, alpha, x, beta, y);
-      else if (U >= 4) nt ? launch_axpy2<4, true>(grid, n2, alpha, x, beta, y) : launch_axpy2<4, false>(grid, n2, alpha, x, beta, y);
-      else nt ? launch_axpy2<2, true>(grid, n2, alpha, x, beta, y) : launch_axpy2<2, false>(grid, n2, alpha, x, beta, y);
-      SPX_LAUNCHED("spx_bs2_axpy");
-    }
-    if (n & 1) {
-      hipLaunchKernelGGL(k_axpy1, dim3(1), dim3(256), 0, current_stream(), n - 1, n, alpha, x, beta, y);
-      SPX_LAUNCHED("spx_bs2_axpy tail");
-    }
+    unsigned grid;  // at least one block
+    int rc = vec_blocks(n2, (U >= 8 ? 8 : U >= 4 ? 4 : 2) * 256, &grid);
+    if (rc) return rc;
+    if (U >= 8) nt ? launch_axpy2<8, true>(grid, n, alpha, x, beta, y) : launch_axpy2<8, false>(grid, n, alpha, x, beta, y);
+    else if (U >= 4) nt ? launch_axpy2<4, true>(grid, n, alpha, x, beta, y) : launch_axpy2<4, false>(grid, n, alpha, x, beta, y);
+    else nt ? launch_axpy2<2, true>(grid, n, alpha, x, beta, y) : launch_axpy2<2, false>(grid, n, alpha, x, beta, y);
+    SPX_LAUNCHED("spx_bs2_axpy");
   } else {
     int64_t g = (n + 255) / 256;
     if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(k_axpy1, dim3((unsigned)g), dim3(256), 0, current_stream(), (int64_t)0, n,
+    hipLaunchKernelGGL(k_axpy1, dim3((unsigned)g), dim3(256), 0, current_stream(), n,
                        alpha, x, beta, y);
     SPX_LAUNCHED("spx_bs2_axpy");
   }
