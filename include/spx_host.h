@@ -35,7 +35,9 @@ typedef struct {
   int32_t kind, unique;
   int64_t NgatherGlobal;
   double setup_seconds;
-  int32_t scatter_by_rows; /* scatter path: 1 row blocks, 0 local order (spxh_ogs_set_scatter_path) */
+  int32_t scatter_by_rows; /* scatter path: 1 row blocks, 0 local order (spxh_ogs_set_scatter_path);
+                              as set up, 1 still sends up to 4 fields in local order, but for
+                              the Trans scatter of a Signed operator */
   int32_t mixed_tiles[2];  /* FP32 / BF16 gather+scatter on tiles of their own (1) or the FP64 one's (0) */
   int32_t gs_nontemporal;  /* spx_srb_t.nontemporal of the Sym gather+scatter's tiles */
 } spxh_ogs_info_t;

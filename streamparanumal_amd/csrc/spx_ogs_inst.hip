@@ -188,25 +188,52 @@ int launch_scatter(const Launch &L, const int *bs, const int *st, const int *ids
   });
 }
 
-int launch_scatter_inv(hipStream_t s, int64_t n, int K, const int *g2l, const T *gv, T *v, int npl) {
-  npl = npl >= 16 ? 16 : (npl >= 8 ? 8 : 4);
-  const int64_t per_block = (int64_t)npl * kThreads;
-  const int64_t blocks = (n + per_block - 1) / per_block;
+// K <= 4 on vectors aligned to 16 bytes (and a map or row vector aligned to its
+// vector load) goes word by word, but for two or three 4-byte fields; the
+// rest, a lane per node.
+int launch_scatter_inv(hipStream_t s, int64_t n, int K, const int *g2l, const T *gv, T *v) {
+  constexpr int kVec = 16 / sizeof(T);
+  constexpr int kPasses = 2, kNodes = 4;  // 16-byte stores / nodes per lane
+  const bool narrow = sizeof(T) == 4 && (K == 2 || K == 3);
+  const bool ntm = n * (int64_t)sizeof(int) > kNtMapBytes;
+  const bool words = K <= 4 && !narrow && aligned(v, 16) && (K > 1 || aligned(g2l, sizeof(int) * kVec)) &&
+                     (K == 1 || K % kVec || aligned(gv, 16));
+  const int64_t per_block = (int64_t)kThreads * (words ? kPasses * kVec : kNodes);
+  const int64_t blocks = ((words ? n * K : n) + per_block - 1) / per_block;
   if (blocks > INT32_MAX) return fail(SPX_ERR_ARG, "spx_ogs_scatter_inverse: n too large");
-  const int kf = (K >= 1 && K <= 4) ? K : 1;
-  const dim3 grid((unsigned)blocks, kf == 1 ? K : 1);
-  auto go = [&](auto npl_c) {
-    constexpr int NPL = decltype(npl_c)::value;
-    switch (kf) {
-      case 1: hipLaunchKernelGGL((k_scatter_inv<T, 1, NPL>), grid, dim3(kThreads), 0, s, n, K, g2l, gv, v); break;
-      case 2: hipLaunchKernelGGL((k_scatter_inv<T, 2, NPL>), grid, dim3(kThreads), 0, s, n, K, g2l, gv, v); break;
-      case 3: hipLaunchKernelGGL((k_scatter_inv<T, 3, NPL>), grid, dim3(kThreads), 0, s, n, K, g2l, gv, v); break;
-      default: hipLaunchKernelGGL((k_scatter_inv<T, 4, NPL>), grid, dim3(kThreads), 0, s, n, K, g2l, gv, v); break;
+  const int kf = K <= 4 ? K : 1;
+  const dim3 grid((unsigned)blocks, words || kf > 1 ? 1 : K);
+  if (words) {
+#define SPX_WORDS(KF, NTM) \
+  hipLaunchKernelGGL((k_scatter_words<T, KF, kPasses, NTM>), grid, dim3(kThreads), 0, s, n, g2l, gv, v)
+    if (K == 1 && ntm) SPX_WORDS(1, true);
+    else if (K == 1) SPX_WORDS(1, false);
+    else if (K == 4) SPX_WORDS(4, false);
+    else if constexpr (sizeof(T) == 8) {
+      if (K == 2) SPX_WORDS(2, false);
+      else SPX_WORDS(3, false);
     }
-  };
-  if (npl == 16) go(std::integral_constant<int, 16>{});
-  else if (npl == 8) go(std::integral_constant<int, 8>{});
-  else go(std::integral_constant<int, 4>{});
+#undef SPX_WORDS
+    return SPX_OK;
+  }
+#define SPX_INV(KF, NT) \
+  hipLaunchKernelGGL((k_scatter_inv<T, KF, kNodes, NT>), grid, dim3(kThreads), 0, s, n, K, g2l, gv, v)
+  if constexpr (sizeof(T) == 4) {
+    if (narrow) {
+      if (K == 2 && ntm) SPX_INV(2, 2);
+      else if (K == 2) SPX_INV(2, 1);
+      else if (ntm) SPX_INV(3, 2);
+      else SPX_INV(3, 1);
+      return SPX_OK;
+    }
+  }
+  switch (kf) {
+    case 1: SPX_INV(1, 0); break;
+    case 2: SPX_INV(2, 0); break;
+    case 3: SPX_INV(3, 0); break;
+    default: SPX_INV(4, 0); break;
+  }
+#undef SPX_INV
   return SPX_OK;
 }
 

@@ -37,6 +37,11 @@ namespace spx {
 namespace ogsk {
 
 constexpr int kThreads = 256;
+constexpr int kXcdLog2Inv = 5;  // local-order scatter: XCD blocks of 32 workgroups
+// Local-order scatter of one field: a map of more bytes is read past the caches.  Of the 256
+// MB that the Infinity Cache holds, a smaller map keeps its part between calls
+// (108 MB: 44 us, 57 non-temporal; 226 MB: 158, 148 non-temporal).
+constexpr int64_t kNtMapBytes = (int64_t)160 << 20;
 
 struct Launch {
   int nblocks;
@@ -919,17 +924,26 @@ __global__ __launch_bounds__(kThreads) void k_scatter(Launch L, const int *__res
 // handles the NPL nodes b*NPL*256 + u*256 + t, so each map load and value
 // store of a wave covers 64 consecutive nodes (a lane taking NPL
 // consecutive nodes instead spread every store of a wave over NPL*64 nodes
-// and ran at 2.6 TB/s).
-template <typename T, int KF, int NPL>
+// and ran at 2.6 TB/s).  NT, where the K = KF values of a wave's 64 nodes are
+// consecutive: as in k_scatter_words below, the stores (1) and the map of a
+// large vector (2) are non-temporal and XCDs take blocks of 32 workgroups.
+// FP32, K = 3, us per call, without / with: 48^3 p=7 238 / 226, 64^3 p=7 597 /
+// 533, 46^3 p=9 428 / 393, 50^3 p=3 32 / 25.
+template <typename T, int KF, int NPL, int NT>
 __global__ __launch_bounds__(kThreads) void k_scatter_inv(int64_t n, int K, const int *__restrict__ g2l,
                                                           const T *__restrict__ gv, T *__restrict__ v) {
   const int kb = blockIdx.y * KF;
-  const int64_t base = (int64_t)blockIdx.x * NPL * kThreads + threadIdx.x;
+  const int b = NT ? xcd_tile(blockIdx.x, gridDim.x, 8, kXcdLog2Inv) : blockIdx.x;
+  const int64_t base = (int64_t)b * NPL * kThreads + threadIdx.x;
   int r[NPL];
 #pragma unroll
   for (int u = 0; u < NPL; ++u) {
     const int64_t l = base + (int64_t)u * kThreads;
-    r[u] = l < n ? g2l[l] : -1;
+    r[u] = -1;
+    if (l < n) {
+      if constexpr (NT == 2) r[u] = __builtin_nontemporal_load(g2l + l);
+      else r[u] = g2l[l];
+    }
   }
   T x[NPL][KF];
 #pragma unroll
@@ -940,7 +954,89 @@ __global__ __launch_bounds__(kThreads) void k_scatter_inv(int64_t n, int K, cons
   for (int u = 0; u < NPL; ++u)
     if (r[u] >= 0)
 #pragma unroll
-      for (int f = 0; f < KF; ++f) v[(base + (int64_t)u * kThreads) * K + kb + f] = x[u][f];
+      for (int f = 0; f < KF; ++f) {
+        T *dst = v + (base + (int64_t)u * kThreads) * K + kb + f;
+        if constexpr (NT > 0) nt_store(x[u][f], dst);
+        else *dst = x[u][f];
+      }
+}
+
+// The same for K = KF <= 4 fields, the vector v taken as n*KF words in order: a
+// lane takes W = 16 / sizeof(T) words next to each other, word i being field
+// i % KF of node i / KF, so every store of a wave is 1 KiB of consecutive
+// 16-byte stores whatever KF (a lane per node instead stores 24 of its
+// wave's 1536 bytes at a time for three FP64 fields; two or three 4-byte
+// fields stay with it, whose node is one 8- or 12-byte store: FP32, K = 3,
+// 64^3 p=7 533 us against 736 in words).  For one field the map
+// entries come in as one vector load; where KF is a multiple of W, the words are
+// one node's and its row's come in as one 16-byte load.
+// The stores are non-temporal: each line is written once, and what is read
+// again, the rows (by every element that shares a node) and a small map, keeps
+// the caches.  NTM: the map is read non-temporally as well, for maps too large
+// to stay there between calls (kNtMapBytes).  Blocks are remapped so that an
+// XCD takes 32 consecutive ones and finds its neighbours' rows in its L2.
+// HBM bounds it: rows once, map and vector once.  Measured on MI355X, us per
+// call: FP64, K = 1, k_scatter_inv / non-temporal stores / and map / and the
+// remap: 48^3 p=7 167 / 159 / 151 / 148 (6.2 TB/s), 64^3 p=7 393 / 377 / 373 /
+// 363, 116^3 p=3 282 / 261 / 258 / 254; map kept, without / with the remap:
+// 50^3 p=3 23.5 / 18.7, 150^3 p=1 47 / 44.  FP64, K = 3, a lane per node /
+// words: 46^3 p=9 868 / 785, 29^3 p=15 948 / 811, 116^3 p=3 966 / 743, 50^3
+// p=3 77 / 43.
+template <typename T, int KF, int PASSES, bool NTM>
+__global__ __launch_bounds__(kThreads) void k_scatter_words(int64_t n, const int *__restrict__ g2l,
+                                                            const T *__restrict__ gv, T *__restrict__ v) {
+  constexpr int W = 16 / sizeof(T);
+  constexpr int R = KF == 1 ? W : KF % W == 0 ? 1 : W;  // map entries per lane and pass
+  typedef int I __attribute__((ext_vector_type(W)));
+  typedef T V __attribute__((ext_vector_type(W)));
+  const int b = xcd_tile(blockIdx.x, gridDim.x, 8, kXcdLog2Inv);
+  const uint64_t words = (uint64_t)n * KF;
+  const uint64_t base = ((uint64_t)b * PASSES * kThreads + threadIdx.x) * W;
+  int r[PASSES][R];
+#pragma unroll
+  for (int u = 0; u < PASSES; ++u) {
+    const uint64_t i = base + (uint64_t)u * kThreads * W;
+    if (KF == 1 && i + W <= words) {
+      const I *m = reinterpret_cast<const I *>(g2l + i);
+      I x;
+      if constexpr (NTM) x = __builtin_nontemporal_load(m);
+      else x = *m;
+#pragma unroll
+      for (int w = 0; w < R; ++w) r[u][w] = x[w];
+    } else {
+#pragma unroll
+      for (int w = 0; w < R; ++w) r[u][w] = i + w < words ? g2l[(i + w) / KF] : -1;
+    }
+  }
+  V x[PASSES];
+#pragma unroll
+  for (int u = 0; u < PASSES; ++u) {
+    const uint64_t i = base + (uint64_t)u * kThreads * W;
+    if constexpr (R == 1) {
+      const int row = r[u][0] < 0 ? 0 : r[u][0];
+      x[u] = *reinterpret_cast<const V *>(gv + (int64_t)row * KF + (int)(i % KF));
+    } else {
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const int row = r[u][w] < 0 ? 0 : r[u][w];
+        x[u][w] = gv[(int64_t)row * KF + (int)((i + w) % KF)];
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < PASSES; ++u) {
+    T *dst = v + base + (uint64_t)u * kThreads * W;
+    bool all = true;
+#pragma unroll
+    for (int w = 0; w < R; ++w) all = all && r[u][w] >= 0;
+    if (all) {
+      __builtin_nontemporal_store(x[u], reinterpret_cast<V *>(dst));
+    } else {
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+        if (r[u][R == 1 ? 0 : w] >= 0) dst[w] = x[u][w];
+    }
+  }
 }
 
 // --------------------------------------------------------------- extract --
@@ -988,7 +1084,7 @@ int launch_gs_sym(const Launch &L, int op, const int *bs, const int *st, const i
   int launch_gather(const Launch &L, int op, const int *bs, const int *st, const int *ids, const T *v, T *gv); \
   int launch_scatter(const Launch &L, const int *bs, const int *st, const int *ids, const T *gv, T *v);    \
   int launch_extract(hipStream_t s, int64_t total, int K, const int *ids, const T *q, T *gq);           \
-  int launch_scatter_inv(hipStream_t s, int64_t n, int K, const int *g2l, const T *gv, T *v, int npl); \
+  int launch_scatter_inv(hipStream_t s, int64_t n, int K, const int *g2l, const T *gv, T *v); \
   int launch_gs_srb(const Launch &L, int op, const SrbArgs &A, T *q, int mode,                              \
                     const unsigned long long *memberN);                                                     \
   int launch_gather_srb(const Launch &L, int op, const SrbArgs &A, const T *v, T *gv, int mode,             \

@@ -174,13 +174,26 @@ class ogsOperator_t {
 
   // Local -> gathered row maps of the T- and N-CSR (-1: in no row), for the
   // scatter in local order (spx_ogs_scatter_inverse), whose stores are
-  // coalesced whatever the rows.  It is the default when rows are short: hex
-  // boxes at ~1e8 nodes, us per call (row blocks / local order): p=1 553 /
-  // 236, p=3 325 / 291, p=5 328 / 288, but p=7 394 / 405 and p=15 326 / 347,
-  // with rows / local nodes 0.13, 0.43, 0.58, 0.68 and 0.83.
+  // coalesced whatever the rows.  A lane per node (the form left to more than 4
+  // fields and unaligned vectors) is the default when rows are short: hex boxes
+  // at ~1e8 nodes, us per call (row blocks / a lane per node): p=1 553 / 236,
+  // p=3 325 / 291, p=5 328 / 288, but p=7 394 / 405 and p=15 326 / 347, with
+  // rows / local nodes 0.13, 0.43, 0.58, 0.68 and 0.83.
   deviceMemory<dlong> o_localRowT, o_localRowN;
   static constexpr double kScatterByRowsMinRatio = 0.63;
   bool scatterByRows = true;  // false: scatter through the local -> row maps
+  bool scatterRowsChosen = false;  // scatterByRows set by the caller: every scatter goes by rows
+
+  // Up to 4 fields to every member go in local order also where rows are long,
+  // unless the caller chose row blocks (or the CSR): their stores are whole 16-byte words
+  // in order.  Row tiles / local order, us per call: FP64 one field 12^3 p=7
+  // 7.0 / 5.2, 48^3 p=7 171 / 150, 64^3 p=7 384 / 361, 29^3 p=15 334 / 293,
+  // 1250^2 Quad p=7 291 / 279; FP32 64^3 p=7 286 / 231.  The N-CSR scatter of a
+  // Signed operator stores to single nodes, and more fields one at a time:
+  // those keep the rule on row length.
+  bool ScatterWords(const Transpose trans, const int k) const {
+    return !scatterRowsChosen && scatterSorted && k <= 4 && (trans != Trans || kind == Unsigned);
+  }
 
   // The non-symmetric gather+scatter stages two value tiles, so its row
   // blocks hold at most min(blockNnz, 2048) entries.

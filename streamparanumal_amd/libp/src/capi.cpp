@@ -210,6 +210,7 @@ int spxh_ogs_set_scatter_path(spxh_ogs_t h, int by_rows) {
     auto op = h->ogs.localOperator();
     LIBP_ABORT("ogs not set up", !op);
     op->scatterByRows = by_rows != 0;
+    op->scatterRowsChosen = by_rows != 0;
   });
 }
 

@@ -406,7 +406,7 @@ void ogsOperator_t::GatherRaw(Type type, Op op, Transpose trans, int k, const vo
 }
 
 void ogsOperator_t::ScatterRaw(Type type, Transpose trans, int k, const void *gv, void *v) {
-  if (!scatterByRows) {
+  if (!scatterByRows || ScatterWords(trans, k)) {
     const dlong nrows = (trans == Trans) ? NrowsN : NrowsT;
     if (nrows && Ncols)
       SPX_CHECK(spx_ogs_scatter_inverse((int)type, k, Ncols, (trans == Trans ? o_localRowN : o_localRowT).ptr(), gv, v));
