@@ -106,6 +106,15 @@ template <typename S> struct FoldWide {
   static __device__ __forceinline__ double init() { return 0.0; }
   static __device__ __forceinline__ void apply(double &a, S x) { a += Store<S>::to_f64(x); }
   static __device__ __forceinline__ S out(double a) { return Store<S>::from_f64(a); }
+  // out(0.0 + x): x itself but for -0 (+0) and a BF16 NaN (the one NaN)
+  static __device__ __forceinline__ S one(S x) {
+    if constexpr (sizeof(S) == 2) {
+      const uint16_t mag = x.bits & 0x7fff;
+      return S{mag > 0x7f80 ? kBf16NaN : mag == 0 ? (uint16_t)0 : x.bits};
+    } else {
+      return out(0.0 + Store<S>::to_f64(x));
+    }
+  }
 };
 
 template <typename S>

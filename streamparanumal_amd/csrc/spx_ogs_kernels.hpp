@@ -66,30 +66,37 @@ template <> struct Lim<int> { static __device__ __forceinline__ int max() { retu
 template <> struct Lim<long long> { static __device__ __forceinline__ long long max() { return LLONG_MAX; } };
 
 // ogsOperator.cpp:37-56 (host) / ogsUtils.cpp:62-103 (device defines).
-// Acc is the accumulator type, out() turns it into the stored result.
+// Acc is the accumulator type, out() turns it into the stored result, one(x)
+// is the stored result of a row of the one member x; it enters another fold
+// as x does (one(one(x)) == one(x), and a sum of one(x) + ... is that of x +
+// ...: only -0 becomes +0, as it does in 0 + x).
 template <typename T, int OP> struct Fold;
 template <typename T> struct Fold<T, SPX_ADD> {
   typedef T Acc;
   static __device__ __forceinline__ T init() { return T(0); }
   static __device__ __forceinline__ void apply(T &a, T b) { a += b; }
+  static __device__ __forceinline__ T one(T x) { return T(0) + x; }
   static __device__ __forceinline__ T out(T a) { return a; }
 };
 template <typename T> struct Fold<T, SPX_MUL> {
   typedef T Acc;
   static __device__ __forceinline__ T init() { return T(1); }
   static __device__ __forceinline__ void apply(T &a, T b) { a *= b; }
+  static __device__ __forceinline__ T one(T x) { return T(1) * x; }
   static __device__ __forceinline__ T out(T a) { return a; }
 };
 template <typename T> struct Fold<T, SPX_MAX> {
   typedef T Acc;
   static __device__ __forceinline__ T init() { return -Lim<T>::max(); }
   static __device__ __forceinline__ void apply(T &a, T b) { a = (b > a) ? b : a; }
+  static __device__ __forceinline__ T one(T x) { return (x > init()) ? x : init(); }
   static __device__ __forceinline__ T out(T a) { return a; }
 };
 template <typename T> struct Fold<T, SPX_MIN> {
   typedef T Acc;
   static __device__ __forceinline__ T init() { return Lim<T>::max(); }
   static __device__ __forceinline__ void apply(T &a, T b) { a = (b < a) ? b : a; }
+  static __device__ __forceinline__ T one(T x) { return (x < init()) ? x : init(); }
   static __device__ __forceinline__ T out(T a) { return a; }
 };
 
@@ -427,6 +434,45 @@ template <typename T> struct GsLds<T, 1, true> {
   __device__ int get_head(int i) const { return (int)((unsigned)e[i].next >> 16); }
 };
 
+// Rows of two or more members, packed into lanes.  A wave owns PER chunks of 64
+// positions; bit j of `lead` says that its position in chunk j leads such a
+// row.  Folding the rows where they start walks each chunk's rows in a loop of
+// its own, with the lanes of the other positions idle; instead the leading
+// positions are first moved into consecutive lanes, in order: chunk j's n of
+// them go to lanes fill .. fill+n-1 (mod 64) by one ds_permute, in which the
+// other lanes' positions take the remaining slots, so every lane receives
+// exactly one word and no LDS is used.  Each full set of 64 is handed on as
+// use(j, h), h the lane's leading position, and the rest as use(PER, h), h = -1
+// in lanes without one.  All lanes of the wave call it; branches are uniform.
+// The packing costs about ten instructions per chunk, and one walk of all
+// fields' rounds pays for it: measured with K = 1, BF16 48^3 p=7 went from 119
+// to 124 us and the FP64 gather of 50^3 p=3 from 26.5 to 27.4.
+template <int PER, int NT, typename Use>
+__device__ __forceinline__ void pack_rows(unsigned lead, Use &&use) {
+  const int t = threadIdx.x, l = t & 63;
+  int cur = -1, fill = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const bool is = (lead >> j) & 1u;
+    const unsigned long long m = __ballot(is);
+    if (m == 0) continue;
+    const int n = (int)__popcll(m);
+    const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    const int to = (fill + (is ? before : n + l - before)) & 63;
+    const int got = __builtin_amdgcn_ds_permute(to << 2, t + j * NT);
+    const int at = (l - fill) & 63;  // lane l holds the at-th of this chunk's
+    if (fill + n < 64) {
+      cur = at < n ? got : cur;
+      fill += n;
+    } else {
+      use(j, l >= fill ? got : cur);
+      fill += n - 64;
+      cur = l < fill ? got : -1;
+    }
+  }
+  if (fill > 0) use(PER, cur);
+}
+
 template <typename T, int OP, int KF, int PER, int NT = kThreads, typename F = Fold<T, OP>, int MODE = kAll,
           bool NTV = false>
 __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restrict__ q,
@@ -470,13 +516,18 @@ __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restri
   const int kb = blockIdx.y * KF;
   const int64_t K = L.K;
   const int t = threadIdx.x;
+  // no next member; with heads beside the links, a row of one member is its own head
+  auto end_link = [&](int i) {
+    if constexpr (kHeadLink) S.set_link_head(i, kEnd, i);
+    else S.set_next(i, kEnd);
+  };
   if (cap >= PER * NT) {  // every slot a position (the usual tile)
 #pragma unroll
-    for (int j = 0; j < PER; ++j) S.set_next(t + j * NT, kEnd);
+    for (int j = 0; j < PER; ++j) end_link(t + j * NT);
   } else {
 #pragma unroll
     for (int j = 0; j < PER; ++j)
-      if (t + j * NT < cap) S.set_next(t + j * NT, kEnd);
+      if (t + j * NT < cap) end_link(t + j * NT);
   }
   int id[PER], prev[PER], row[PER];
   unsigned valid;
@@ -513,26 +564,78 @@ __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restri
     if (((valid >> j) & 1u) && (unsigned)prev[j] < (unsigned)cap) S.set_next(prev[j], t + j * NT);
   // one LDS round per field (one round in all for KF == 1 and word-major)
   constexpr int ROUNDS = kWord ? 1 : KF;
+  // Several rounds on tiles of 8 positions or more per lane pack the leading
+  // positions (pack_rows), once for all rounds.  Measured, us per call, without /
+  // with: FP32 values, K = 3, 48x47x46 p=4 83.6 / 79.0, a batch of 16 uneven
+  // boxes with its CG update 378 / 369; small operators' tiles of 4 positions
+  // per lane lose (FP32, K = 2, 172224-node Tri p=1 5.4 / 5.8).
+  constexpr bool kPack = KF > 1 && PER >= 8;
+  int heads[kPack && ROUNDS > 1 ? PER + 1 : 1];
+  unsigned sets = 0;
+  (void)heads;
+  (void)sets;
+  // folds the row led by position h, field f0's round; walks end at kEnd (>
+  // cap), and the step bound also ends them on a malformed layout
+  auto fold_row = [&](int h, int f0) {
+    if constexpr (kHeadLink) {
+      // several fields, one per round: the first round's walk also
+      // writes the head's position beside each member's link, and every
+      // round's members read the row value from the head
+      typename F::Acc acc = F::init();
+      for (int i = h, s = 0; i < cap && s < cap; ++s) {
+        int n;
+        F::apply(acc, S.get_both(i, 0, n));
+        if (f0 == 0) S.set_link_head(i, n, h);
+        i = n;
+      }
+      S.set_val(h, 0, F::out(acc));
+    } else {
+      // every field held in LDS in one walk, and one more writes the row's values
+      typename F::Acc acc[LF];
+#pragma unroll
+      for (int f = 0; f < LF; ++f) acc[f] = F::init();
+      for (int i = h, s = 0; i < cap && s < cap; ++s) {
+#pragma unroll
+        for (int f = 0; f < LF; ++f) F::apply(acc[f], S.get_val(i, f));
+        i = S.get_next(i);
+      }
+      T r[LF];
+#pragma unroll
+      for (int f = 0; f < LF; ++f) r[f] = F::out(acc[f]);
+      for (int i = h, s = 0; i < cap && s < cap; ++s) {
+#pragma unroll
+        for (int f = 0; f < LF; ++f) S.set_val(i, f, r[f]);
+        i = S.get_next(i);
+      }
+    }
+  };
 #pragma unroll
   for (int f0 = 0; f0 < ROUNDS; ++f0) {
     if (f0 > 0) __syncthreads();  // the previous field has been read back
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       if constexpr (!kWord) {
-        if ((valid >> j) & 1u) S.set_val(t + j * NT, 0, v[j][f0]);
+        if ((valid >> j) & 1u) {
+          // packed rows have two members or more: a row's first member
+          // enters as the row of one member it may be
+          if (kPack && prev[j] < 0) S.set_val(t + j * NT, 0, F::one(v[j][f0]));
+          else S.set_val(t + j * NT, 0, v[j][f0]);
+        }
       } else {
         const unsigned long long vm = __ballot((valid >> j) & 1u);
+        const unsigned long long hm = __ballot(prev[j] < 0);
 #pragma unroll
         for (int f = 0; f < KF; ++f) {
-          const int w = f * 64 + l;
-          if ((vm >> (w / KF)) & 1ull) vals[(cb0 + j * NT) * KF + w] = v[j][f];
+          const int w = f * 64 + l, pos = w / KF;
+          if ((vm >> pos) & 1ull)
+            vals[(cb0 + j * NT) * KF + w] = kPack && ((hm >> pos) & 1ull) ? F::one(v[j][f]) : v[j][f];
         }
       }
     }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PER; ++j)
-      if (((valid >> j) & 1u) && prev[j] < 0) {
+      if (!kPack && ((valid >> j) & 1u) && prev[j] < 0) {
         const int h = t + j * NT;
         if constexpr (KF == 1) {
           // One walk: each member's link, once read, is replaced by the head's
@@ -548,35 +651,31 @@ __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restri
             i = n;
           }
           S.set_val(h, 0, F::out(acc));
-        } else if constexpr (kHeadLink) {
-          // several fields, one per round: the first round's walk also
-          // writes the head's position beside each member's link, and every
-          // round's members read the row value from the head
-          typename F::Acc acc = F::init();
-          for (int i = h, s = 0; i < cap && s < cap; ++s) {
-            int n;
-            F::apply(acc, S.get_both(i, 0, n));
-            if (f0 == 0) S.set_link_head(i, n, h);
-            i = n;
-          }
-          S.set_val(h, 0, F::out(acc));
         } else {
-#pragma unroll
-          for (int f = 0; f < LF; ++f) {
-            typename F::Acc acc = F::init();
-            for (int i = h, s = 0; i < cap && s < cap; ++s) {
-              int n;
-              F::apply(acc, S.get_both(i, f, n));
-              i = n;
-            }
-            const T r = F::out(acc);
-            for (int i = h, s = 0; i < cap && s < cap; ++s) {
-              S.set_val(i, f, r);
-              i = S.get_next(i);
-            }
-          }
+          fold_row(h, f0);
         }
       }
+    if constexpr (kPack) {
+      if (f0 == 0) {
+        unsigned lead = 0;  // leading positions whose row goes on
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+          if (((valid >> j) & 1u) && prev[j] < 0 && S.get_next(t + j * NT) < cap) lead |= 1u << j;
+        pack_rows<PER, NT>(lead, [&](int s, int h) {
+          if constexpr (ROUNDS > 1) {
+            heads[s] = h;
+            sets |= 1u << s;
+          } else if (h >= 0) {
+            fold_row(h, 0);
+          }
+        });
+      }
+      if constexpr (ROUNDS > 1) {
+#pragma unroll
+        for (int s = 0; s <= PER; ++s)
+          if (((sets >> s) & 1u) && heads[s] >= 0) fold_row(heads[s], f0);
+      }
+    }
     __syncthreads();
     if constexpr (kHeadLink) {
 #pragma unroll
