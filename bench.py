@@ -40,18 +40,18 @@ BIN = os.path.join(ROOT, "streamparanumal_amd", "bin")
 KERNEL_PATTERNS = {
     "BS1_copy": r"k_copy2<4, true>",
     "BS2_axpy": r"k_axpy2<",
-    "BS3_norm_reference": r"k_red_ref1<0, \d+, \d+, \w+, false>",
-    "BS4_dot_reference": r"k_red_ref1<1, \d+, \d+, \w+, false>",
-    "BS5_cg_update_reference": r"k_red_ref1<2, \d+, \d+, \w+, false>",
-    "BS5_cg_full_reference": r"k_red_ref1<3, \d+, \d+, \w+, false>",
-    "BS3_norm_fast": r"k_red_ref1<0, \d+, \d+, \w+, true>",
-    "BS4_dot_fast": r"k_red_ref1<1, \d+, \d+, \w+, true>",
-    "BS5_cg_update_fast": r"k_red_ref1<2, \d+, \d+, \w+, true>",
-    "BS5_cg_full_fast": r"k_red_ref1<3, \d+, \d+, \w+, true>",
+    "BS3_norm_reference": r"k_red_ref1<0, \d+, \d+, \w+, false, \w+>",
+    "BS4_dot_reference": r"k_red_ref1<1, \d+, \d+, \w+, false, \w+>",
+    "BS5_cg_update_reference": r"k_red_ref1<2, \d+, \d+, \w+, false, \w+>",
+    "BS5_cg_full_reference": r"k_red_ref1<3, \d+, \d+, \w+, false, \w+>",
+    "BS3_norm_fast": r"k_red_ref1<0, \d+, \d+, \w+, true, \w+>",
+    "BS4_dot_fast": r"k_red_ref1<1, \d+, \d+, \w+, true, \w+>",
+    "BS5_cg_update_fast": r"k_red_ref1<2, \d+, \d+, \w+, true, \w+>",
+    "BS5_cg_full_fast": r"k_red_ref1<3, \d+, \d+, \w+, true, \w+>",
     "BS5_cg_full_f32": r"k_cg_mixed1<float",
     "BS5_cg_full_bf16": r"k_cg_mixed1<[^>]*bf16_t",
     "BS6_gather": r"k_gather_srb<double",
-    "BS7_scatter": r"k_scatter_srb<double",
+    "BS7_scatter": r"k_scatter_words<double",
     "BS8_gather_scatter": r"k_gs_srb<double",
     "BS8_gather_scatter_f32": r"k_gs_srb<float",
     "BS8_gather_scatter_bf16": r"k_gs_srb<[^,]*bf16_t",
