@@ -342,7 +342,7 @@ template <bool FAST> __device__ __forceinline__ double small_stage2(const double
 
 template <int KIND, bool COMP>
 __global__ __launch_bounds__(64 * kSmallWaves) void k_red_small(int64_t n, int nb, RedArgs A,
-                                                                double *__restrict__ out) {
+                                                                double *__restrict__ tmp, double *__restrict__ out) {
   __shared__ double part[256];
   constexpr int G = KIND == RED_CGFULL ? 2 : 4;  // blocks of a wave whose loads are in flight together
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -357,7 +357,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_red_small(int64_t n, int n
       double v = (e[0].value() + e[2].value()) + (e[1].value() + e[3].value());
 #pragma unroll
       for (int w = 32; w >= 1; w >>= 1) v += __shfl_down(v, w, 64);
-      if (l == 0 && b + g < nb) part[b + g] = v;
+      if (l == 0 && b + g < nb) {
+        part[b + g] = v;
+        tmp[b + g] = v;  // the caller's partials hold what stage 1 leaves there
+      }
     }
   }
   __syncthreads();
@@ -493,7 +496,7 @@ static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *
     if (nb > bs) nb = bs;
     if (bs == 256 && n <= small_n(KIND)) {
       hipLaunchKernelGGL((k_red_small<KIND, false>), dim3(1), dim3(64 * kSmallWaves), 0, current_stream(), n, (int)nb,
-                         A, out);
+                         A, tmp, out);
       SPX_LAUNCHED(name);
       return SPX_OK;
     }
@@ -521,7 +524,7 @@ static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *
   const int64_t grid = fast_grid();
   if (n <= small_n(KIND) && nb <= grid && nb <= 256) {
     hipLaunchKernelGGL((k_red_small<KIND, true>), dim3(1), dim3(64 * kSmallWaves), 0, current_stream(), n, (int)nb, A,
-                       out);
+                       tmp, out);
     SPX_LAUNCHED(name);
     return SPX_OK;
   }
