@@ -256,12 +256,9 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
 // same launch shape and element order with compensated lane sums, so it runs
 // at the reference order's bandwidth and is more accurate.
 // TAIL: the entries past a lane's last whole group of U also go out in groups
-// instead of one memory latency each.  That is taken while a lane has fewer
-// than kTailGroups whole groups (n < 2^25 at 256 x 256 lanes); measured on
-// MI355X, full form, us per call, one by one / in groups: n = 500001 8.6 / 7.3,
-// 900000 11.4 / 10.9, 2000001 23.1 / 20.1, 3000003 31.8 / 28.7, 10000001 89.4 /
-// 87.2, but 2^27 1094 / 1105 (norm, dot and update there within 0.3 %).
-constexpr int kTailGroups = 32;
+// instead of one memory latency each.  Taken by the full form on 256-entry
+// blocks only (tail_groups below): its six streams per entry are what the
+// latencies cost.
 template <int KIND, int BS, int U, bool NT, bool COMP, bool TAIL>
 __global__ __launch_bounds__(BS) void k_red_ref1(int64_t n, int64_t nblock, RedArgs A,
                                                  double *__restrict__ partials) {
@@ -439,14 +436,30 @@ static int fast_grid() {
   return g < 1 ? 1 : (g > kFastGridMax ? kFastGridMax : g);
 }
 
+// Grouped tails for the full form on 256-entry blocks, from two and a half
+// entries per lane (fewer: the group that may reach past n only adds its bounds) to 32
+// groups (above: n >= 2^25 at 256 x 256 lanes, where the tail is under 3 % of
+// the work).  Measured on MI355X, us per call in a replayed graph, one by one / in
+// groups: n = 65537 4.6 / 5.1, 131073 4.7 / 5.0, 180000 5.2 / 4.8, 250000 5.8 / 5.0,
+// 500001 8.2 / 7.5, 2000001 22.0 / 19.9, 7000003 64.8 / 62.9, 2^24-1 147.6 / 147.4.  The others keep
+// their entries one by one: dot 900000 5.7 / 6.2, 2^24-1 40.7 / 42.2, update
+// 900000 6.3 / 7.0, and on wider blocks, whose lanes have few entries (2000001,
+// 1024-entry blocks: dot 7.4 / 9.3, update 9.1 / 11.4, full form 21.0 / 23.3;
+// 512: dot 6.3 / 7.9).
+template <int KIND, int BS> constexpr bool kTailGroups = KIND == RED_CGFULL && BS == 256;
+static bool tail_groups(int64_t n, int64_t lanes, int U) { return 2 * n >= 5 * lanes && n < 32 * U * lanes; }
+
 template <int KIND, int BS, int U, bool NT, bool COMP>
 static void launch_ref1_u(int64_t n, int64_t nb, const RedArgs &A, double *tmp) {
-  if (n < (int64_t)kTailGroups * U * BS * nb)
-    hipLaunchKernelGGL((k_red_ref1<KIND, BS, U, NT, COMP, true>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
-                       nb, A, tmp);
-  else
-    hipLaunchKernelGGL((k_red_ref1<KIND, BS, U, NT, COMP, false>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
-                       nb, A, tmp);
+  if constexpr (kTailGroups<KIND, BS>) {
+    if (tail_groups(n, BS * nb, U)) {
+      hipLaunchKernelGGL((k_red_ref1<KIND, BS, U, NT, COMP, true>), dim3((unsigned)nb), dim3(BS), 0, current_stream(),
+                         n, nb, A, tmp);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_red_ref1<KIND, BS, U, NT, COMP, false>), dim3((unsigned)nb), dim3(BS), 0, current_stream(), n,
+                     nb, A, tmp);
 }
 template <int KIND, int BS, bool NT, bool COMP>
 static void launch_ref1_nt(int64_t n, int64_t nb, const RedArgs &A, double *tmp, int unroll) {
