@@ -209,8 +209,10 @@ template <> struct LaneSum<true> {
 template <bool C> __device__ __forceinline__ LaneSum<C> &lane_of(LaneSum<C> &a, int) { return a; }
 template <bool C, int N> __device__ __forceinline__ LaneSum<C> &lane_of(LaneSum<C> (&a)[N], int u) { return a[u]; }
 
-// LAST: the group may reach past n; entries there are neither loaded, stored
-// nor added.
+// LAST: the group may reach past n.  Entries there are neither loaded nor
+// stored and add +0, which changes no sum (sums start from +0 and are never -0):
+// leaving the loop at the first of them instead put every add behind its own
+// branch (one-launch FAST update of 5000 entries 7.9 us against 5.0).
 template <int KIND, int U, bool NT, bool LAST = false, typename ACC>
 __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t stride, ACC &acc, int64_t n = 0) {
   double va[U], vb[U], vr[U], vx[U];
@@ -218,21 +220,23 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t i = id + u * stride;
-    if (LAST && i >= n) break;
-    if constexpr (KIND == RED_CGFULL) {
-      ix[u] = x_index(A, i);
-      va[u] = ldv<NT>(A.a + ix[u]);
-    } else {
-      va[u] = ldv<NT>(A.a + i);
+    va[u] = vb[u] = vr[u] = vx[u] = 0.0;
+    if constexpr (KIND == RED_CGFULL) ix[u] = x_index(A, i);
+    if (!LAST || i < n) {
+      if constexpr (KIND == RED_CGFULL) {
+        va[u] = ldv<NT>(A.a + ix[u]);
+        vx[u] = ldv<NT>(A.x + ix[u]);
+      } else {
+        va[u] = ldv<NT>(A.a + i);
+      }
+      if constexpr (KIND == RED_DOT || KIND == RED_CGFULL) vb[u] = ldv<NT>(A.b + i);
+      if constexpr (KIND == RED_CG || KIND == RED_CGFULL) vr[u] = ldv<NT>(A.r + i);
     }
-    if constexpr (KIND == RED_DOT || KIND == RED_CGFULL) vb[u] = ldv<NT>(A.b + i);
-    if constexpr (KIND == RED_CG || KIND == RED_CGFULL) vr[u] = ldv<NT>(A.r + i);
-    if constexpr (KIND == RED_CGFULL) vx[u] = ldv<NT>(A.x + ix[u]);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t i = id + u * stride;
-    if (LAST && i >= n) break;
+    const bool in = !LAST || i < n;
     double term;
     if constexpr (KIND == RED_NORM) {
       term = va[u] * va[u];
@@ -240,15 +244,17 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
       term = va[u] * vb[u];
     } else if constexpr (KIND == RED_CG) {
       const double rr = vr[u] + A.alpha * va[u];
-      stv<NT>(A.r + i, rr);
+      if (in) stv<NT>(A.r + i, rr);
       term = rr * rr;
     } else {
-      stv<NT>(A.x + ix[u], vx[u] + A.alpha * va[u]);
       const double rr = vr[u] - A.alpha * vb[u];
-      stv<NT>(A.r + i, rr);
+      if (in) {
+        stv<NT>(A.x + ix[u], vx[u] + A.alpha * va[u]);
+        stv<NT>(A.r + i, rr);
+      }
       term = rr * rr;
     }
-    lane_of(acc, u).add(term);
+    lane_of(acc, u).add(in ? term : 0.0);
   }
 }
 
