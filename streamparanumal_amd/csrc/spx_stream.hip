@@ -309,7 +309,7 @@ __global__ __launch_bounds__(BS) void k_red_ref2(int64_t nblock, const double *_
 }
 
 
-// Both stages in one workgroup, for 256-entry blocks with n <= small_n(KIND): each
+// Both stages in one workgroup, for 256-entry blocks with n up to small_n: each
 // lane of the two-launch form then has one entry, so a wave takes whole
 // blocks, 4 entries of each per lane, and the tree's steps are register adds (128, 64)
 // and lane shifts (32 .. 2, s[0]+s[1]) in the same order; the partials stay in
@@ -496,11 +496,39 @@ static spx_tuning_t reference_tuning(int kind) {
 
 // Largest n of the one-launch form (at most 256 * 256).  One workgroup's
 // loads and stores run through one CU, so the line lies where that costs as
-// much as the second launch.  Measured on MI355X, us per call back to back,
-// two launches / one: norm n = 2500 6.3 / 3.7, 16384 6.6 / 4.6; dot 2500 6.5 /
-// 3.9, 16384 6.8 / 6.2; update 5000 6.6 / 5.1, 10007 6.9 / 6.6, 16000 6.9 /
-// 8.3; full form 2500 6.8 / 4.6, 5000 7.0 / 5.9, 10007 6.8 / 8.7.
-constexpr int64_t small_n(int kind) { return kind == RED_CGFULL ? 5120 : kind == RED_CG ? 8192 : 16384; }
+// much as the second launch: about 2.9 us of host time launch by launch, and about
+// 1.5 us in a replayed graph, so a captured call has a lower one (FAST mode,
+// whose compensated folds add to the workgroup's time, none).  Measured on
+// MI355X, us per call, two launches / one:
+//   launch by launch (FAST: one): norm n = 2500 5.9 / 3.7 (3.8), 16384 5.8 / 4.7
+//   (5.4); dot 5000 5.9 / 4.2 (5.0), 8192 5.9 / 4.6 (5.2), 12000 5.9 / 5.6 (6.3),
+//   16384 5.9 / 6.5; update 5000 6.0 / 4.8 (5.6), 7000 6.0 / 5.4 (6.2), 8192 6.0 /
+//   5.4; full form 3500 6.1 / 4.8 (5.3), 5000 6.1 / 5.9 (6.5)
+//   replayed: norm 8192 4.0 / 3.6 (4.3), 10007 3.9 / 4.0; dot 4500 4.2 / 4.0, 5000 4.0
+//   / 4.2, 1500 4.1 / 3.2 (3.9), 10007 3.9 / 5.1; update 3000 4.2 / 4.1, 5000 4.0 /
+//   4.9 (5.6); full form 2500 4.3 / 4.3, 5000 4.3 / 5.9 (6.5)
+constexpr int64_t small_n(int kind, bool fast) {
+  switch (kind) {
+    case RED_NORM: return 16384;
+    case RED_DOT: return fast ? 8192 : 12288;
+    case RED_CG: return fast ? 5120 : 8192;
+    default: return fast ? 3584 : 5120;
+  }
+}
+constexpr int64_t small_n_captured(int kind, bool fast) {
+  if (fast) return 0;
+  return kind == RED_NORM ? 8192 : kind == RED_DOT ? 4096 : kind == RED_CG ? 3072 : 2560;
+}
+static bool one_launch(int kind, bool fast, int64_t n) {
+  if (n > small_n(kind, fast)) return false;
+  if (n <= small_n_captured(kind, fast)) return true;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(current_stream(), &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st == hipStreamCaptureStatusNone;
+}
 
 template <int KIND>
 static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *tmp, double *out,
@@ -513,7 +541,7 @@ static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *
       return fail(SPX_ERR_ARG, std::string(name) + ": block_size must be 256, 512 or 1024");
     int64_t nb = (n + bs - 1) / bs;
     if (nb > bs) nb = bs;
-    if (bs == 256 && n <= small_n(KIND)) {
+    if (bs == 256 && one_launch(KIND, false, n)) {
       hipLaunchKernelGGL((k_red_small<KIND, false>), dim3(1), dim3(64 * kSmallWaves), 0, current_stream(), n, (int)nb,
                          A, tmp, out);
       SPX_LAUNCHED(name);
@@ -541,7 +569,7 @@ static int run_reduction(const char *name, int64_t n, const RedArgs &A, double *
   // partials; deterministic for a given grid.
   int64_t nb = (n + 255) / 256;
   const int64_t grid = fast_grid();
-  if (n <= small_n(KIND) && nb <= grid && nb <= 256) {
+  if (nb <= grid && nb <= 256 && one_launch(KIND, true, n)) {
     hipLaunchKernelGGL((k_red_small<KIND, true>), dim3(1), dim3(64 * kSmallWaves), 0, current_stream(), n, (int)nb, A,
                        tmp, out);
     SPX_LAUNCHED(name);
