@@ -35,9 +35,9 @@ typedef struct {
   int32_t kind, unique;
   int64_t NgatherGlobal;
   double setup_seconds;
-  int32_t scatter_by_rows; /* scatter path: 1 row blocks, 0 local order (spxh_ogs_set_scatter_path);
-                              as set up, 1 still sends up to 4 fields in local order, but for
-                              the Trans scatter of a Signed operator */
+  int32_t scatter_by_rows; /* 1: rows are long enough (or the caller chose) to scatter by rows, 0: local
+                              order.  spxh_ogs_scatter_path says which way a scatter goes and
+                              what the caller chose. */
   int32_t mixed_tiles[2];  /* FP32 / BF16 gather+scatter on tiles of their own (1) or the FP64 one's (0) */
   int32_t gs_nontemporal;  /* spx_srb_t.nontemporal of the Sym gather+scatter's tiles */
 } spxh_ogs_info_t;
@@ -83,11 +83,19 @@ int spxh_ogs_copy_csr(spxh_ogs_t ogs, int which, int32_t *rowStarts, int32_t *co
    blocks, and gather+scatter blocks */
 int spxh_ogs_set_block_nnz(spxh_ogs_t ogs, int32_t block_nnz);
 int spxh_ogs_set_gs_block_nnz(spxh_ogs_t ogs, int32_t block_nnz);
-/* scatter path: 1 = over the row blocks (ogsKernels.okl scatter), 0 =
-   through the local->row map in local order; results are identical.  The
+/* scatter path: 1 (any positive value) = over the row blocks
+   (ogsKernels.okl scatter), 0 = through the local->row map in local order,
+   negative = as set up; results are identical.  The
    setup picks local order when the operator has fewer than 0.63 rows per
-   local entry (short rows: there its coalesced stores win), else rows. */
+   local entry (short rows: there its coalesced stores win), else rows, of which up
+   to 4 fields still go in local order, but for the Trans scatter of a Signed
+   operator.  A negative value also returns the rows to the layout set up
+   (spxh_ogs_set_gather_format). */
 int spxh_ogs_set_scatter_path(spxh_ogs_t ogs, int by_rows);
+/* *chosen: the last value given to spxh_ogs_set_scatter_path as -1, 0 or 1 (-1 if none),
+   which restores it; *runs: the way of a scatter of k fields, 0 = T- or
+   N-CSR row blocks, 1 = sorted-run row blocks, 2 = local order. */
+int spxh_ogs_scatter_path(spxh_ogs_t ogs, int trans, int k, int32_t *chosen, int32_t *runs);
 /* layout of the Sym gather+scatter: 1 = sorted-run row blocks (spx_srb_t, the
    default), 0 = the T-CSR row blocks; results are identical.  xcd_remap is the
    sorted-run launch hint (negative: library default, 0 hardware order, 1 remap in

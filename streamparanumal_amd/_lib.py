@@ -153,6 +153,7 @@ SPXH_FUNCS = {
     "spxh_ogs_copy_csr": (C.c_int, [vp, C.c_int, vp, vp, vp]),
     "spxh_ogs_set_block_nnz": (C.c_int, [vp, i32]),
     "spxh_ogs_set_gs_block_nnz": (C.c_int, [vp, i32]),
+    "spxh_ogs_scatter_path": (C.c_int, [vp, C.c_int, C.c_int, C.POINTER(i32), C.POINTER(i32)]),
     "spxh_ogs_set_scatter_path": (C.c_int, [vp, C.c_int]),
     "spxh_ogs_global_to_local": (C.c_int, [vp, vp]),
     "spxh_ogs_gather_scatter": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, C.c_int, vp]),

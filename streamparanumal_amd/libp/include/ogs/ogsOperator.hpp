@@ -182,7 +182,12 @@ class ogsOperator_t {
   deviceMemory<dlong> o_localRowT, o_localRowN;
   static constexpr double kScatterByRowsMinRatio = 0.63;
   bool scatterByRows = true;  // false: scatter through the local -> row maps
-  bool scatterRowsChosen = false;  // scatterByRows set by the caller: every scatter goes by rows
+  bool scatterByRowsSetup = true;  // what the setup picked for it
+  // the caller's choice of the path: 1 row blocks, 0 local order, -1 none
+  // (scatterByRowsSetup, and ScatterWords)
+  int scatterChosen = -1;
+  void SetScatterByRows(bool byRows) { scatterByRows = scatterByRowsSetup = byRows; }  // the setup's
+  void ChooseScatterPath(int path);
 
   // Up to 4 fields to every member go in local order also where rows are long,
   // unless the caller chose row blocks (or the CSR): their stores are whole 16-byte words
@@ -192,8 +197,12 @@ class ogsOperator_t {
   // Signed operator stores to single nodes, and more fields one at a time:
   // those keep the rule on row length.
   bool ScatterWords(const Transpose trans, const int k) const {
-    return !scatterRowsChosen && scatterSorted && k <= 4 && (trans != Trans || kind == Unsigned);
+    return scatterChosen < 0 && scatterSorted && k <= 4 && (trans != Trans || kind == Unsigned);
   }
+
+  // the path that ScatterRaw takes
+  enum ScatterPath { ScatterRowBlocks = 0, ScatterTiles = 1, ScatterLocal = 2 };
+  ScatterPath PathOfScatter(const Transpose trans, const int k) const;
 
   // The non-symmetric gather+scatter stages two value tiles, so its row
   // blocks hold at most min(blockNnz, 2048) entries.

@@ -209,8 +209,18 @@ int spxh_ogs_set_scatter_path(spxh_ogs_t h, int by_rows) {
   return guarded([&] {
     auto op = h->ogs.localOperator();
     LIBP_ABORT("ogs not set up", !op);
-    op->scatterByRows = by_rows != 0;
-    op->scatterRowsChosen = by_rows != 0;
+    op->ChooseScatterPath(by_rows);
+  });
+}
+
+int spxh_ogs_scatter_path(spxh_ogs_t h, int trans, int k, int32_t *chosen, int32_t *runs) {
+  if (!h || !chosen || !runs) return err(SPX_ERR_ARG, "spxh_ogs_scatter_path: null");
+  if (trans < 0 || trans > 2 || k < 1) return err(SPX_ERR_ARG, "spxh_ogs_scatter_path: trans must be 0..2 and k positive");
+  return guarded([&] {
+    auto op = h->ogs.localOperator();
+    LIBP_ABORT("ogs not set up", !op);
+    *chosen = op->scatterChosen;
+    *runs = (int32_t)op->PathOfScatter((ogs::Transpose)trans, k);
   });
 }
 

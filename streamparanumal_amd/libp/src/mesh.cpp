@@ -232,7 +232,7 @@ void mesh_t::BoxGatherScatterSetup(ogs::ogs_t &ogs, int type, dlong nx, dlong ny
   // triangles' simplex node order leaves short runs at every degree: their
   // scatter runs in local order (p=7, ~1e8 nodes: 323 -> 304 us), which the
   // row ratio alone does not pick at p=7 (0.68 rows per node)
-  if (type == TRIANGLES) ogs.localOperator()->scatterByRows = false;
+  if (type == TRIANGLES) ogs.localOperator()->SetScatterByRows(false);
   // gather+scatter tiles over blocks of the node lattice (the ids are lattice
   // ids, 1 + gx + gy*Gx [+ gz*Gx*Gy]) where that measured faster on MI355X at
   // ~1e8 nodes, us per call: Quad p=3 379 -> 347 and Tri p=3 394 -> 368 with

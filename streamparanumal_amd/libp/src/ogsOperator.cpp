@@ -80,7 +80,7 @@ ogsOperator_t::ogsOperator_t(platform_t &platform_, Kind kind_, const dlong Nrow
   };
   o_localRowT = localRows(NrowsT, rowStartsT, colIdsT);
   o_localRowN = (kind == Signed) ? localRows(NrowsN, rowStartsN, colIdsN) : o_localRowT;
-  scatterByRows = NrowsT >= kScatterByRowsMinRatio * Ncols;
+  SetScatterByRows(NrowsT >= kScatterByRowsMinRatio * Ncols);
 }
 
 void ogsOperator_t::SetGsBlockNnz(int nnz) {
@@ -405,15 +405,30 @@ void ogsOperator_t::GatherRaw(Type type, Op op, Transpose trans, int k, const vo
   }
 }
 
+// A chosen path is scatterByRows itself; none (-1) is the state after setup, the
+// row layout's (scatterSorted) included.
+void ogsOperator_t::ChooseScatterPath(int path) {
+  scatterChosen = path < 0 ? -1 : path != 0;
+  scatterByRows = path < 0 ? scatterByRowsSetup : path != 0;
+  if (path < 0) scatterSorted = true;
+}
+
+ogsOperator_t::ScatterPath ogsOperator_t::PathOfScatter(const Transpose trans, const int k) const {
+  if (!scatterByRows || ScatterWords(trans, k)) return ScatterLocal;
+  const bool srbRows = NgsBlocks && rowSrb.rowsAscending;  // the layout numbers the rows
+  const bool tiles = scatterSorted && srbRows && (trans != Trans || signedSrb || kind == Unsigned);
+  return tiles ? ScatterTiles : ScatterRowBlocks;
+}
+
 void ogsOperator_t::ScatterRaw(Type type, Transpose trans, int k, const void *gv, void *v) {
-  if (!scatterByRows || ScatterWords(trans, k)) {
+  const ScatterPath path = PathOfScatter(trans, k);
+  if (path == ScatterLocal) {
     const dlong nrows = (trans == Trans) ? NrowsN : NrowsT;
     if (nrows && Ncols)
       SPX_CHECK(spx_ogs_scatter_inverse((int)type, k, Ncols, (trans == Trans ? o_localRowN : o_localRowT).ptr(), gv, v));
     return;
   }
-  const bool srbRows = NgsBlocks && rowSrb.rowsAscending;  // the layout numbers the rows
-  if (trans == Trans && scatterSorted && srbRows && (signedSrb || kind == Unsigned)) {
+  if (trans == Trans && path == ScatterTiles) {
     const spx_srb_t d = rowSrb.Device();
     if (kind == Unsigned) SPX_CHECK(spx_ogs_scatter_srb((int)type, k, &d, gv, v));
     else SPX_CHECK(spx_ogs_scatter_srb_signed((int)type, k, &d, rowSrb.DeviceMemberN(), NrowsN, gv, v));
@@ -421,7 +436,7 @@ void ogsOperator_t::ScatterRaw(Type type, Transpose trans, int k, const void *gv
     if (NrowBlocksN)
       SPX_CHECK(spx_ogs_scatter((int)type, k, NrowBlocksN, o_blockRowStartsN.ptr(), o_rowStartsN.ptr(),
                                 o_colIdsN.ptr(), blockNnz, gv, v));
-  } else if (trans != Trans && scatterSorted && srbRows) {
+  } else if (path == ScatterTiles) {
     const spx_srb_t d = rowSrb.Device();
     SPX_CHECK(spx_ogs_scatter_srb((int)type, k, &d, gv, v));
   } else {

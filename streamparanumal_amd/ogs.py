@@ -355,8 +355,17 @@ class Ogs:
         return {f: getattr(best, f) for f, _ in _lib.GsTuning._fields_}
 
     def set_scatter_path(self, by_rows):
-        """Scatter over the CSR row blocks (True, default) or through the local->row map (False)."""
-        checkh(libspxhost().spxh_ogs_set_scatter_path(self.h, 1 if by_rows else 0), "spxh_ogs_set_scatter_path")
+        """Scatter over the row blocks (True), through the local->row map (False), or as set up (None, the
+        default: by rows where they are long, up to 4 fields of them in local order too)."""
+        checkh(libspxhost().spxh_ogs_set_scatter_path(self.h, -1 if by_rows is None else 1 if by_rows else 0),
+               "spxh_ogs_set_scatter_path")
+
+    def scatter_path(self, k=1, trans=_lib.NOTRANS):
+        """(chosen, runs): the path given to set_scatter_path (None, True or False), which restores it, and
+        the way a scatter of k fields goes: "rows" (CSR), "tiles" (sorted-run rows) or "local"."""
+        c, r = _lib.i32(), _lib.i32()
+        checkh(libspxhost().spxh_ogs_scatter_path(self.h, trans, k, C.byref(c), C.byref(r)), "spxh_ogs_scatter_path")
+        return None if c.value < 0 else bool(c.value), ("rows", "tiles", "local")[r.value]
 
     def global_to_local(self):
         """SetupGlobalToLocalMapping (ogsSetup.cpp:833-849): the T-row of every local node, -1 where
