@@ -130,7 +130,9 @@ int spxh_ogs_set_gs_mixed_tiles(spxh_ogs_t ogs, int storage, const int64_t *keys
 int spxh_ogs_set_gs_nontemporal(spxh_ogs_t ogs, int mode);
 /* layouts of the T-CSR gather (Trans) and scatter (NoTrans): 1 = the
    sorted-run blocks of the gather+scatter, 0 = T-CSR row blocks, -1 = keep;
-   both sorted by default.  Results are identical. */
+   both sorted by default.  A scatter layout given here holds for every
+   scatter that goes by rows, up to 4 fields included, until
+   spxh_ogs_set_scatter_path is given a negative value.  Results are identical. */
 int spxh_ogs_set_gather_format(spxh_ogs_t ogs, int gather_sorted, int scatter_sorted);
 /* Autotuner (no reference counterpart; the reference's ogs::Auto times its
    halo exchange methods, ogsSetup.cpp:116-125, the same way): times every

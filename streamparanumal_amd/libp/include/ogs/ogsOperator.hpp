@@ -188,16 +188,17 @@ class ogsOperator_t {
   int scatterChosen = -1;
   void SetScatterByRows(bool byRows) { scatterByRows = scatterByRowsSetup = byRows; }  // the setup's
   void ChooseScatterPath(int path);
+  bool scatterFormatChosen = false;  // scatterSorted set by the caller: rows go on that layout
 
   // Up to 4 fields to every member go in local order also where rows are long,
-  // unless the caller chose row blocks (or the CSR): their stores are whole 16-byte words
+  // unless the caller chose row blocks or a layout of them: their stores are whole 16-byte words
   // in order.  Row tiles / local order, us per call: FP64 one field 12^3 p=7
   // 7.0 / 5.2, 48^3 p=7 171 / 150, 64^3 p=7 384 / 361, 29^3 p=15 334 / 293,
   // 1250^2 Quad p=7 291 / 279; FP32 64^3 p=7 286 / 231.  The N-CSR scatter of a
   // Signed operator stores to single nodes, and more fields one at a time:
   // those keep the rule on row length.
   bool ScatterWords(const Transpose trans, const int k) const {
-    return scatterChosen < 0 && scatterSorted && k <= 4 && (trans != Trans || kind == Unsigned);
+    return scatterChosen < 0 && !scatterFormatChosen && k <= 4 && (trans != Trans || kind == Unsigned);
   }
 
   // the path that ScatterRaw takes

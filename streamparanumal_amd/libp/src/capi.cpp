@@ -358,7 +358,10 @@ int spxh_ogs_set_gather_format(spxh_ogs_t h, int gather_sorted, int scatter_sort
     auto op = h->ogs.localOperator();
     LIBP_ABORT("ogs not set up", !op);
     if (gather_sorted >= 0) op->gatherSorted = gather_sorted != 0;
-    if (scatter_sorted >= 0) op->scatterSorted = scatter_sorted != 0;
+    if (scatter_sorted >= 0) {
+      op->scatterSorted = scatter_sorted != 0;
+      op->scatterFormatChosen = true;
+    }
   });
 }
 

@@ -410,7 +410,10 @@ void ogsOperator_t::GatherRaw(Type type, Op op, Transpose trans, int k, const vo
 void ogsOperator_t::ChooseScatterPath(int path) {
   scatterChosen = path < 0 ? -1 : path != 0;
   scatterByRows = path < 0 ? scatterByRowsSetup : path != 0;
-  if (path < 0) scatterSorted = true;
+  if (path < 0) {
+    scatterSorted = true;
+    scatterFormatChosen = false;
+  }
 }
 
 ogsOperator_t::ScatterPath ogsOperator_t::PathOfScatter(const Transpose trans, const int k) const {

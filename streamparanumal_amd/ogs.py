@@ -337,7 +337,8 @@ class Ogs:
 
     def set_gather_format(self, gather_sorted=None, scatter_sorted=None):
         """T-CSR gather (Trans) and scatter (NoTrans) on the sorted-run blocks (True) or the T-CSR row
-        blocks (False); None keeps the current choice (both sorted by default)."""
+        blocks (False); None keeps the current choice (both sorted by default).  A scatter layout chosen
+        here holds for up to 4 fields too, until set_scatter_path(None)."""
         enc = lambda x: -1 if x is None else (1 if x else 0)
         checkh(libspxhost().spxh_ogs_set_gather_format(self.h, enc(gather_sorted), enc(scatter_sorted)),
                "spxh_ogs_set_gather_format")

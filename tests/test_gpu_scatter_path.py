@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 import streamparanumal_amd as spx
-from streamparanumal_amd import ogs
+from streamparanumal_amd import device, ogs
 from streamparanumal_amd.device import DeviceArray
 
 pytestmark = pytest.mark.gpu
@@ -38,10 +38,11 @@ def test_automatic_path_and_the_way_back(dev, oracle):
         assert g.scatter_path()[0] is choice and ways() == [[way] * 3] * 2
         g.set_scatter_path(before)  # what was saved restores it
         assert g.scatter_path()[0] is None and ways() == auto
-    g.set_gather_format(None, False)
-    assert ways() == [["rows"] * 3] * 2
-    g.set_scatter_path(None)
-    assert ways() == auto
+    for fmt, way in ((False, "rows"), (True, "tiles")):
+        g.set_gather_format(None, fmt)
+        assert ways() == [[way] * 3] * 2
+        g.set_scatter_path(None)
+        assert ways() == auto
 
 
 def test_short_rows(dev, oracle):
@@ -61,3 +62,34 @@ def test_triangles_scatter_in_local_order(dev):
     for choice in (None, True, None):
         g.set_scatter_path(choice)
         assert g.scatter_path(5)[1] == ("tiles" if choice else "local")
+
+
+DTYPES = [np.float32, np.float64, np.int32, np.int64]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("lanes,cap", [(64, 256), (64, 512), (256, 2048), (256, 700)])
+@pytest.mark.parametrize("mesh", [LONG, SHORT])
+def test_scatter_on_tiles_and_rows(dev, oracle, mesh, lanes, cap, dtype):
+    """The sorted-run scatter and the CSR's, by name, on one-wave and full tiles."""
+    print("[case] scatter on tiles", mesh, lanes, cap, np.dtype(dtype).name, flush=True)
+    ids = ogs.hex_ids(*mesh)
+    g, o = ogs.Ogs(ids), oracle.Ogs(ids)
+    g.set_block_nnz(2048, gs_cap=cap)
+    device.set_tuning("ogs_gs_srb", variant=2 if lanes == 64 else 0)
+    try:
+        for fmt, way in ((True, "tiles"), (False, "rows")):
+            g.set_scatter_path(True)
+            g.set_gather_format(None, fmt)
+            for k in (1, 2, 3, 4, 5):
+                for trans in (spx.NOTRANS, spx.TRANS):
+                    rows = g.NlocalP if trans == spx.TRANS else g.NlocalT
+                    src = np.floor(oracle.uniform(rows * k, 21) * 1000).astype(dtype)
+                    base = np.floor(oracle.uniform(g.N * k, 22) * 1000).astype(dtype)
+                    assert g.scatter_path(k, trans)[1] == way
+                    dv = DeviceArray.from_numpy(base)
+                    g.scatter(dv, DeviceArray.from_numpy(src), k, trans)
+                    device.check_kernel_errors()
+                    assert np.array_equal(dv.to_numpy(), o.scatter(src, base, k, trans)), (k, trans, way)
+    finally:
+        device.set_tuning("ogs_gs_srb", variant=-1)
