@@ -216,6 +216,12 @@ int spx_ogs_gather_scatter(int type, int op, int K, int32_t nblocks, const int32
    the reference's GlobalToLocal (ogsSetup.cpp:833-849).  gv must hold at
    least one row (K values) even if every map entry is -1. */
 int spx_ogs_scatter_inverse(int type, int K, int32_t n, const int32_t *g2l, const void *gv, void *v);
+/* 1 if that call would store whole 16-byte words (up to 4 fields, v aligned
+   to 16 bytes, and g2l (one field) or gv (nodes of whole words) aligned to
+   the words it reads) or nodes of two or three 4-byte fields, non-temporally;
+   0 if a lane per node and field with ordinary stores, which long rows
+   leave to the row blocks. */
+int spx_ogs_scatter_inverse_streams(int type, int K, const int32_t *g2l, const void *gv, const void *v);
 /* extract (ogsKernels.okl:167-177): gq[k + n*K] = q[k + ids[n]*K], n < n_ids */
 int spx_ogs_extract(int type, int K, int32_t n_ids, const int32_t *ids, const void *q, void *gq);
 

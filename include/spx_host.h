@@ -89,13 +89,16 @@ int spxh_ogs_set_gs_block_nnz(spxh_ogs_t ogs, int32_t block_nnz);
    setup picks local order when the operator has fewer than 0.63 rows per
    local entry (short rows: there its coalesced stores win), else rows, of which up
    to 4 fields still go in local order, but for the Trans scatter of a Signed
-   operator.  A negative value also returns the rows to the layout set up
+   operator and for vectors whose alignment leaves whole words out
+   (spx_ogs_scatter_inverse_streams).  A negative value also returns the rows to the layout set up
    (spxh_ogs_set_gather_format). */
 int spxh_ogs_set_scatter_path(spxh_ogs_t ogs, int by_rows);
 /* *chosen: the last value given to spxh_ogs_set_scatter_path as -1, 0 or 1 (-1 if none),
-   which restores it; *runs: the way of a scatter of k fields, 0 = T- or
-   N-CSR row blocks, 1 = sorted-run row blocks, 2 = local order. */
-int spxh_ogs_scatter_path(spxh_ogs_t ogs, int trans, int k, int32_t *chosen, int32_t *runs);
+   which restores it; *runs: the way of a scatter of k fields from gv to
+   v, 0 = T- or N-CSR row blocks, 1 = sorted-run row blocks, 2 = local order.
+   Only the alignment of gv and v counts (NULL: aligned). */
+int spxh_ogs_scatter_path(spxh_ogs_t ogs, int type, int trans, int k, const void *gv, const void *v,
+                          int32_t *chosen, int32_t *runs);
 /* layout of the Sym gather+scatter: 1 = sorted-run row blocks (spx_srb_t, the
    default), 0 = the T-CSR row blocks; results are identical.  xcd_remap is the
    sorted-run launch hint (negative: library default, 0 hardware order, 1 remap in

@@ -124,6 +124,7 @@ SPX_FUNCS = {
     "spx_ogs_gather": (C.c_int, [C.c_int, C.c_int, C.c_int, i32, vp, vp, vp, i32, vp, vp]),
     "spx_ogs_scatter": (C.c_int, [C.c_int, C.c_int, i32, vp, vp, vp, i32, vp, vp]),
     "spx_ogs_gather_scatter": (C.c_int, [C.c_int, C.c_int, C.c_int, i32, vp, i32, vp, vp, i32, vp, vp, i32, vp]),
+    "spx_ogs_scatter_inverse_streams": (C.c_int, [C.c_int, C.c_int, vp, vp, vp]),
     "spx_ogs_scatter_inverse": (C.c_int, [C.c_int, C.c_int, i32, vp, vp, vp]),
     "spx_ogs_extract": (C.c_int, [C.c_int, C.c_int, i32, vp, vp, vp]),
     "spx_ogs_gather_scatter_srb": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(Srb), vp]),
@@ -153,7 +154,7 @@ SPXH_FUNCS = {
     "spxh_ogs_copy_csr": (C.c_int, [vp, C.c_int, vp, vp, vp]),
     "spxh_ogs_set_block_nnz": (C.c_int, [vp, i32]),
     "spxh_ogs_set_gs_block_nnz": (C.c_int, [vp, i32]),
-    "spxh_ogs_scatter_path": (C.c_int, [vp, C.c_int, C.c_int, C.POINTER(i32), C.POINTER(i32)]),
+    "spxh_ogs_scatter_path": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, vp, vp, C.POINTER(i32), C.POINTER(i32)]),
     "spxh_ogs_set_scatter_path": (C.c_int, [vp, C.c_int]),
     "spxh_ogs_global_to_local": (C.c_int, [vp, vp]),
     "spxh_ogs_gather_scatter": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, C.c_int, vp]),

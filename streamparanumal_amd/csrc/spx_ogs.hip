@@ -295,6 +295,14 @@ int spx_ogs_scatter_srb_signed(int type, int K, const spx_srb_t *srb, const uint
   return SPX_OK;
 }
 
+int spx_ogs_scatter_inverse_streams(int type, int K, const int32_t *g2l, const void *gv, const void *v) {
+  if (!type_size(type) || K < 1) return 0;
+  return by_type(type, [&](auto *tp) {
+    using T = std::remove_pointer_t<decltype(tp)>;
+    return scatter_inv_streams(K, g2l, (const T *)gv, (const T *)v) ? 1 : 0;
+  });
+}
+
 int spx_ogs_scatter_inverse(int type, int K, int32_t n, const int32_t *g2l, const void *gv, void *v) {
   SPX_NEED_DEVICE();
   if (!type_size(type)) return fail(SPX_ERR_ARG, "spx_ogs_scatter_inverse: unknown type");

@@ -188,16 +188,29 @@ int launch_scatter(const Launch &L, const int *bs, const int *st, const int *ids
   });
 }
 
+// Two or three 4-byte fields: a node is one 8- or 12-byte store of its lane,
+// whatever the alignment.
+static bool scatter_narrow(int K) { return sizeof(T) == 4 && (K == 2 || K == 3); }
+
 // K <= 4 on vectors aligned to 16 bytes (and a map or row vector aligned to its
 // vector load) goes word by word, but for two or three 4-byte fields; the
 // rest, a lane per node.
+static bool scatter_words(int K, const int *g2l, const T *gv, const T *v) {
+  constexpr int kVec = 16 / sizeof(T);
+  return K <= 4 && !scatter_narrow(K) && aligned(v, 16) && (K > 1 || aligned(g2l, sizeof(int) * kVec)) &&
+         (K == 1 || K % kVec || aligned(gv, 16));
+}
+
+bool scatter_inv_streams(int K, const int *g2l, const T *gv, const T *v) {
+  return scatter_narrow(K) || scatter_words(K, g2l, gv, v);
+}
+
 int launch_scatter_inv(hipStream_t s, int64_t n, int K, const int *g2l, const T *gv, T *v) {
   constexpr int kVec = 16 / sizeof(T);
   constexpr int kPasses = 2, kNodes = 4;  // 16-byte stores / nodes per lane
-  const bool narrow = sizeof(T) == 4 && (K == 2 || K == 3);
+  const bool narrow = scatter_narrow(K);
   const bool ntm = n * (int64_t)sizeof(int) > kNtMapBytes;
-  const bool words = K <= 4 && !narrow && aligned(v, 16) && (K > 1 || aligned(g2l, sizeof(int) * kVec)) &&
-                     (K == 1 || K % kVec || aligned(gv, 16));
+  const bool words = scatter_words(K, g2l, gv, v);
   const int64_t per_block = (int64_t)kThreads * (words ? kPasses * kVec : kNodes);
   const int64_t blocks = ((words ? n * K : n) + per_block - 1) / per_block;
   if (blocks > INT32_MAX) return fail(SPX_ERR_ARG, "spx_ogs_scatter_inverse: n too large");

@@ -1184,6 +1184,7 @@ int launch_gs_sym(const Launch &L, int op, const int *bs, const int *st, const i
   int launch_scatter(const Launch &L, const int *bs, const int *st, const int *ids, const T *gv, T *v);    \
   int launch_extract(hipStream_t s, int64_t total, int K, const int *ids, const T *q, T *gq);           \
   int launch_scatter_inv(hipStream_t s, int64_t n, int K, const int *g2l, const T *gv, T *v); \
+  bool scatter_inv_streams(int K, const int *g2l, const T *gv, const T *v); \
   int launch_gs_srb(const Launch &L, int op, const SrbArgs &A, T *q, int mode,                              \
                     const unsigned long long *memberN);                                                     \
   int launch_gather_srb(const Launch &L, int op, const SrbArgs &A, const T *v, T *gv, int mode,             \

@@ -197,13 +197,18 @@ class ogsOperator_t {
   // 1250^2 Quad p=7 291 / 279; FP32 64^3 p=7 286 / 231.  The N-CSR scatter of a
   // Signed operator stores to single nodes, and more fields one at a time:
   // those keep the rule on row length.
-  bool ScatterWords(const Transpose trans, const int k) const {
-    return scatterChosen < 0 && !scatterFormatChosen && k <= 4 && (trans != Trans || kind == Unsigned);
+  // So do unaligned vectors, but for those whose stores need no alignment
+  // (spx_ogs_scatter_inverse_streams): a lane per node loses there, FP64 one
+  // field 8 bytes off, us per call (row tiles / a lane per node): 30^3 p=9 97.7 / 103,
+  // 10^3 p=15 14.3 / 16.1, FP32 30^3 p=9 53.5 / 66.
+  bool ScatterWords(const Type type, const Transpose trans, const int k, const void *gv, const void *v) const {
+    return scatterChosen < 0 && !scatterFormatChosen && k <= 4 && (trans != Trans || kind == Unsigned) &&
+           spx_ogs_scatter_inverse_streams((int)type, k, (trans == Trans ? o_localRowN : o_localRowT).ptr(), gv, v);
   }
 
   // the path that ScatterRaw takes
   enum ScatterPath { ScatterRowBlocks = 0, ScatterTiles = 1, ScatterLocal = 2 };
-  ScatterPath PathOfScatter(const Transpose trans, const int k) const;
+  ScatterPath PathOfScatter(const Type type, const Transpose trans, const int k, const void *gv, const void *v) const;
 
   // The non-symmetric gather+scatter stages two value tiles, so its row
   // blocks hold at most min(blockNnz, 2048) entries.

@@ -204,6 +204,13 @@ int spxh_ogs_set_gs_block_nnz(spxh_ogs_t h, int32_t nnz) {
   });
 }
 
+static int check_enums(int type, int op, int trans) {
+  if (type < 0 || type > 3) return err(SPX_ERR_ARG, "type must be 0..3 (Float, Double, Int32, Int64)");
+  if (op < 0 || op > 3) return err(SPX_ERR_ARG, "op must be 0..3 (Add, Mul, Max, Min)");
+  if (trans < 0 || trans > 2) return err(SPX_ERR_ARG, "trans must be 0..2 (Sym, NoTrans, Trans)");
+  return SPX_OK;
+}
+
 int spxh_ogs_set_scatter_path(spxh_ogs_t h, int by_rows) {
   if (!h) return err(SPX_ERR_ARG, "spxh_ogs_set_scatter_path: null");
   return guarded([&] {
@@ -213,14 +220,16 @@ int spxh_ogs_set_scatter_path(spxh_ogs_t h, int by_rows) {
   });
 }
 
-int spxh_ogs_scatter_path(spxh_ogs_t h, int trans, int k, int32_t *chosen, int32_t *runs) {
+int spxh_ogs_scatter_path(spxh_ogs_t h, int type, int trans, int k, const void *gv, const void *v, int32_t *chosen,
+                          int32_t *runs) {
   if (!h || !chosen || !runs) return err(SPX_ERR_ARG, "spxh_ogs_scatter_path: null");
-  if (trans < 0 || trans > 2 || k < 1) return err(SPX_ERR_ARG, "spxh_ogs_scatter_path: trans must be 0..2 and k positive");
+  if (int rc = check_enums(type, 0, trans)) return rc;
+  if (k < 1) return err(SPX_ERR_ARG, "spxh_ogs_scatter_path: k must be positive");
   return guarded([&] {
     auto op = h->ogs.localOperator();
     LIBP_ABORT("ogs not set up", !op);
     *chosen = op->scatterChosen;
-    *runs = (int32_t)op->PathOfScatter((ogs::Transpose)trans, k);
+    *runs = (int32_t)op->PathOfScatter((ogs::Type)type, (ogs::Transpose)trans, k, gv, v);
   });
 }
 
@@ -372,13 +381,6 @@ int spxh_ogs_global_to_local(spxh_ogs_t h, int32_t *g2l) {
     h->ogs.SetupGlobalToLocalMapping(m);
     std::copy(m.ptr(), m.ptr() + h->ogs.N, g2l);
   });
-}
-
-static int check_enums(int type, int op, int trans) {
-  if (type < 0 || type > 3) return err(SPX_ERR_ARG, "type must be 0..3 (Float, Double, Int32, Int64)");
-  if (op < 0 || op > 3) return err(SPX_ERR_ARG, "op must be 0..3 (Add, Mul, Max, Min)");
-  if (trans < 0 || trans > 2) return err(SPX_ERR_ARG, "trans must be 0..2 (Sym, NoTrans, Trans)");
-  return SPX_OK;
 }
 
 int spxh_ogs_gather_scatter(spxh_ogs_t h, int type, int op, int trans, int k, void *v) {

@@ -416,15 +416,16 @@ void ogsOperator_t::ChooseScatterPath(int path) {
   }
 }
 
-ogsOperator_t::ScatterPath ogsOperator_t::PathOfScatter(const Transpose trans, const int k) const {
-  if (!scatterByRows || ScatterWords(trans, k)) return ScatterLocal;
+ogsOperator_t::ScatterPath ogsOperator_t::PathOfScatter(const Type type, const Transpose trans, const int k,
+                                                        const void *gv, const void *v) const {
+  if (!scatterByRows || ScatterWords(type, trans, k, gv, v)) return ScatterLocal;
   const bool srbRows = NgsBlocks && rowSrb.rowsAscending;  // the layout numbers the rows
   const bool tiles = scatterSorted && srbRows && (trans != Trans || signedSrb || kind == Unsigned);
   return tiles ? ScatterTiles : ScatterRowBlocks;
 }
 
 void ogsOperator_t::ScatterRaw(Type type, Transpose trans, int k, const void *gv, void *v) {
-  const ScatterPath path = PathOfScatter(trans, k);
+  const ScatterPath path = PathOfScatter(type, trans, k, gv, v);
   if (path == ScatterLocal) {
     const dlong nrows = (trans == Trans) ? NrowsN : NrowsT;
     if (nrows && Ncols)

@@ -361,11 +361,13 @@ class Ogs:
         checkh(libspxhost().spxh_ogs_set_scatter_path(self.h, -1 if by_rows is None else 1 if by_rows else 0),
                "spxh_ogs_set_scatter_path")
 
-    def scatter_path(self, k=1, trans=_lib.NOTRANS):
+    def scatter_path(self, k=1, trans=_lib.NOTRANS, dtype=np.float64, gv=None, v=None):
         """(chosen, runs): the path given to set_scatter_path (None, True or False), which restores it, and
-        the way a scatter of k fields goes: "rows" (CSR), "tiles" (sorted-run rows) or "local"."""
+        the way a scatter of k fields of dtype goes: "rows" (CSR), "tiles" (sorted-run rows) or "local".
+        gv, v: addresses, whose alignment counts (None: aligned)."""
         c, r = _lib.i32(), _lib.i32()
-        checkh(libspxhost().spxh_ogs_scatter_path(self.h, trans, k, C.byref(c), C.byref(r)), "spxh_ogs_scatter_path")
+        checkh(libspxhost().spxh_ogs_scatter_path(self.h, ogs_type(np.dtype(dtype)), trans, k, gv, v, C.byref(c), C.byref(r)),
+               "spxh_ogs_scatter_path")
         return None if c.value < 0 else bool(c.value), ("rows", "tiles", "local")[r.value]
 
     def global_to_local(self):

@@ -4,6 +4,7 @@ import pytest
 
 import streamparanumal_amd as spx
 from streamparanumal_amd import device, ogs
+from streamparanumal_amd._lib import checkh, libspxhost
 from streamparanumal_amd.device import DeviceArray
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +94,29 @@ def test_scatter_on_tiles_and_rows(dev, oracle, mesh, lanes, cap, dtype):
                     assert np.array_equal(dv.to_numpy(), o.scatter(src, base, k, trans)), (k, trans, way)
     finally:
         device.set_tuning("ogs_gs_srb", variant=-1)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+def test_unaligned_vectors_of_long_rows(dev, oracle, dtype, k):
+    """Vectors off a 16-byte boundary keep the row tiles, but for two or three 4-byte fields."""
+    print("[case] unaligned scatter of long rows", np.dtype(dtype).name, k, flush=True)
+    ids = ogs.hex_ids(*LONG)
+    g, o = ogs.Ogs(ids), oracle.Ogs(ids)
+    size = np.dtype(dtype).itemsize
+    src = np.floor(oracle.uniform(g.NlocalT * k, 21) * 1000).astype(dtype)
+    base = np.floor(oracle.uniform(g.N * k, 22) * 1000).astype(dtype)
+    want = o.scatter(src, base, k, spx.NOTRANS)
+    dg, dv = DeviceArray(src.size + 4, dtype), DeviceArray(base.size + 4, dtype)
+    for og in range(16 // size):
+        for ov in range(16 // size):
+            dg.copy_from(np.concatenate([np.zeros(og, dtype), src, np.zeros(4 - og, dtype)]))
+            dv.copy_from(np.concatenate([np.zeros(ov, dtype), base, np.zeros(4 - ov, dtype)]))
+            way = g.scatter_path(k, spx.NOTRANS, dtype, dg.offset(og), dv.offset(ov))[1]
+            # og: a node of whole 16-byte words (K * size a multiple of 16) is read in them
+            words = ov == 0 and (og == 0 or k * size % 16 != 0)
+            assert way == ("local" if words or (size == 4 and k in (2, 3)) else "tiles"), (og, ov)
+            checkh(libspxhost().spxh_ogs_scatter(g.h, device.ogs_type(np.dtype(dtype)), spx.NOTRANS, k, dg.offset(og),
+                                                 dv.offset(ov)), "scatter")
+            device.check_kernel_errors()
+            assert np.array_equal(dv.to_numpy()[ov:ov + base.size], want), (og, ov)
