@@ -473,8 +473,15 @@ __device__ __forceinline__ void pack_rows(unsigned lead, Use &&use) {
   if (fill > 0) use(PER, cur);
 }
 
+// Several rounds on tiles of 8 positions or more per lane pack the leading
+// positions (pack_rows), once for all rounds.  Measured, us per call, without /
+// with: FP32 values, K = 3, 48x47x46 p=4 83.6 / 79.0, a batch of 16 uneven
+// boxes with its CG update 378 / 369; small operators' tiles of 4 positions
+// per lane lose (FP32, K = 2, 172224-node Tri p=1 5.4 / 5.8).
+template <int KF, int PER> constexpr bool kPackRows = KF > 1 && PER >= 8;
+
 template <typename T, int OP, int KF, int PER, int NT = kThreads, typename F = Fold<T, OP>, int MODE = kAll,
-          bool NTV = false>
+          bool NTV = false, bool PACK = kPackRows<KF, PER>>
 __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restrict__ q,
                                                const unsigned long long *__restrict__ memberN) {
   // Several 4- or 8-byte fields per pass: each lane loads and stores its
@@ -516,9 +523,9 @@ __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restri
   const int kb = blockIdx.y * KF;
   const int64_t K = L.K;
   const int t = threadIdx.x;
-  // no next member; with heads beside the links, a row of one member is its own head
+  // no next member; with heads beside the links, a packed tile's row of one member is its own head
   auto end_link = [&](int i) {
-    if constexpr (kHeadLink) S.set_link_head(i, kEnd, i);
+    if constexpr (kHeadLink && PACK) S.set_link_head(i, kEnd, i);
     else S.set_next(i, kEnd);
   };
   if (cap >= PER * NT) {  // every slot a position (the usual tile)
@@ -564,12 +571,7 @@ __global__ __launch_bounds__(NT) void k_gs_srb(Launch L, SRB_PARAMS, T *__restri
     if (((valid >> j) & 1u) && (unsigned)prev[j] < (unsigned)cap) S.set_next(prev[j], t + j * NT);
   // one LDS round per field (one round in all for KF == 1 and word-major)
   constexpr int ROUNDS = kWord ? 1 : KF;
-  // Several rounds on tiles of 8 positions or more per lane pack the leading
-  // positions (pack_rows), once for all rounds.  Measured, us per call, without /
-  // with: FP32 values, K = 3, 48x47x46 p=4 83.6 / 79.0, a batch of 16 uneven
-  // boxes with its CG update 378 / 369; small operators' tiles of 4 positions
-  // per lane lose (FP32, K = 2, 172224-node Tri p=1 5.4 / 5.8).
-  constexpr bool kPack = KF > 1 && PER >= 8;
+  constexpr bool kPack = PACK;
   int heads[kPack && ROUNDS > 1 ? PER + 1 : 1];
   unsigned sets = 0;
   (void)heads;
