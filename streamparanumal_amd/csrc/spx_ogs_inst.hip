@@ -98,6 +98,16 @@ static bool srb_nontemporal(const Launch &W) {
   return (W.ntMask >> e) & 1;
 }
 
+// Trans of two 4-byte fields on tiles of whole memory lines (the Sym pass's
+// non-temporal tiles of 8-byte nodes; hex p = 7 and 15) walks rows where they start:
+// two rounds on such tiles do not pay for the packing.  FP32, us per call, packed / in
+// place: p=7 20^3 23.4 / 22.9, 28^3 43.7 / 41.3, 36^3 89.4 / 85.6, 44^3 182 / 168, p=15 7^3
+// 12.7 / 12.1, 10^3 20.5 / 20.7, 16^3 56.0 / 54.5; on other tiles packing gains
+// (60^3 p=2 32.9 / 38.1, 24^3 p=9 the same).  The Sym and NoTrans passes differ by
+// at most 4 % on line tiles, either way from size to size, and stay packed.
+template <int KF> constexpr bool kTransInPlace = KF == 2 && sizeof(T) == 4;
+[[maybe_unused]] static bool trans_in_place(const Launch &W) { return W.kf == W.K && ((W.ntMask >> 3) & 1); }
+
 // mode (kAll, kFoldN, kStoreN) and memberN: the N-CSR forms, on 256-lane
 // tiles only (one instance set per mode).
 int launch_gs_srb(const Launch &L, int op, const SrbArgs &A, T *q, int mode, const unsigned long long *memberN) {
@@ -112,9 +122,17 @@ int launch_gs_srb(const Launch &L, int op, const SrbArgs &A, T *q, int mode, con
         else if (mode == kFoldN)
           hipLaunchKernelGGL((k_gs_srb<T, OPC, KF, PER, kThreads, Fold<T, OPC>, kFoldN>), grid_of(W),
                              dim3(kThreads), lds, W.stream, W, SRB_ARGS(A), q, memberN);
-        else if (mode == kStoreN)
+        else if (mode == kStoreN) {
+          if constexpr (kTransInPlace<KF> && kPackRows<KF, PER>) {
+            if (trans_in_place(W)) {
+              hipLaunchKernelGGL((k_gs_srb<T, OPC, KF, PER, kThreads, Fold<T, OPC>, kStoreN, false, false>), grid_of(W),
+                                 dim3(kThreads), lds, W.stream, W, SRB_ARGS(A), q, memberN);
+              return SPX_OK;
+            }
+          }
           hipLaunchKernelGGL((k_gs_srb<T, OPC, KF, PER, kThreads, Fold<T, OPC>, kStoreN>), grid_of(W),
                              dim3(kThreads), lds, W.stream, W, SRB_ARGS(A), q, memberN);
+        }
         else if (wave)
           hipLaunchKernelGGL((k_gs_srb<T, OPC, KF, PER, 64>), grid_of(W), dim3(64), lds, W.stream, W, SRB_ARGS(A),
                              q, nullptr);
