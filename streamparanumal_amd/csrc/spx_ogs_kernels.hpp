@@ -38,9 +38,15 @@ namespace ogsk {
 
 constexpr int kThreads = 256;
 constexpr int kXcdLog2Inv = 5;  // local-order scatter: XCD blocks of 32 workgroups
-// Local-order scatter of one field: a map of more bytes is read past the caches.  Of the 256
-// MB that the Infinity Cache holds, a smaller map keeps its part between calls
-// (108 MB: 44 us, 57 non-temporal; 226 MB: 158, 148 non-temporal).
+// Local-order scatter of one field, or of two or three 4-byte ones: a map of more bytes
+// is read past the caches.  Of the 256 MB that the Infinity Cache holds, a
+// smaller map keeps its part between calls.  Measured on MI355X, us per call,
+// map cached / non-temporal, hex p=7: FP64 one field 43 MiB 31.1 / 32.7, 107 78.5 /
+// 78.4, 125 92.1 / 90.0, 166 125 / 122, 216 163 / 159; FP32 43 MiB 19.8 / 21.6, 125
+// 54.9 / 56.7, 166 76.2 / 73.6, 216 102 / 96; two FP32 fields 43 MiB 31.4 / 33.0,
+// 125 93.1 / 91.2, 216 164 / 163; three, whose rows and vector crowd the map out
+// earlier, 43 MiB 42.6 / 43.9, 77 80.6 / 77.5, 125 133 / 125, 216 231 / 232; p=3, one
+// FP64 field, 125 MiB 85.1 / 87.6, 178 127 / 111.
 constexpr int64_t kNtMapBytes = (int64_t)160 << 20;
 
 struct Launch {
@@ -1078,8 +1084,8 @@ __global__ __launch_bounds__(kThreads) void k_scatter_inv(int64_t n, int K, cons
 // XCD takes 32 consecutive ones and finds its neighbours' rows in its L2.
 // HBM bounds it: rows once, map and vector once.  Measured on MI355X, us per
 // call: FP64, K = 1, k_scatter_inv / non-temporal stores / and map / and the
-// remap: 48^3 p=7 167 / 159 / 151 / 148 (6.2 TB/s), 64^3 p=7 393 / 377 / 373 /
-// 363, 116^3 p=3 282 / 261 / 258 / 254; map kept, without / with the remap:
+// remap: 48^3 p=7 167 / 159 / 151 / 148 (0.99 GB: 6.7 TB/s), 64^3 p=7 393 / 377 / 373 /
+// 363, 116^3 p=3 282 / 261 / 258 / 254; map cached, without / with the remap:
 // 50^3 p=3 23.5 / 18.7, 150^3 p=1 47 / 44.  FP64, K = 3, a lane per node /
 // words: 46^3 p=9 868 / 785, 29^3 p=15 948 / 811, 116^3 p=3 966 / 743, 50^3
 // p=3 77 / 43.

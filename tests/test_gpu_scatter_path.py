@@ -4,7 +4,7 @@ import pytest
 
 import streamparanumal_amd as spx
 from streamparanumal_amd import device, ogs
-from streamparanumal_amd._lib import checkh, libspxhost
+from streamparanumal_amd._lib import check, checkh, libspx, libspxhost
 from streamparanumal_amd.device import DeviceArray
 
 pytestmark = pytest.mark.gpu
@@ -120,3 +120,18 @@ def test_unaligned_vectors_of_long_rows(dev, oracle, dtype, k):
                                                  dv.offset(ov)), "scatter")
             device.check_kernel_errors()
             assert np.array_equal(dv.to_numpy()[ov:ov + base.size], want), (og, ov)
+
+
+@pytest.mark.parametrize("k", [2, 3])
+def test_large_map_of_several_narrow_fields(dev, k):
+    """Two and three 4-byte fields through a map past the size that is read non-temporally, ragged end and holes."""
+    n = (160 << 18) + 5
+    print("[case] scatter of narrow fields, large map", n, k, flush=True)
+    g2l = (np.arange(n, dtype=np.int64) * 7919 % 100003).astype(np.int32)
+    g2l[::1009] = -1
+    gv = np.arange(100003 * k, dtype=np.float32)
+    dv, dm, dg = (DeviceArray.from_numpy(a) for a in (np.full(n * k, -7.0, np.float32), g2l, gv))
+    check(libspx().spx_ogs_scatter_inverse(spx.FLOAT, k, n, dm.ptr, dg.ptr, dv.ptr), "scatter")
+    want = gv.reshape(-1, k)[np.maximum(g2l, 0)]
+    want[g2l < 0] = -7.0
+    assert np.array_equal(dv.to_numpy().reshape(-1, k), want)
