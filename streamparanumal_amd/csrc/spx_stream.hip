@@ -209,12 +209,53 @@ template <> struct LaneSum<true> {
 template <bool C> __device__ __forceinline__ LaneSum<C> &lane_of(LaneSum<C> &a, int) { return a; }
 template <bool C, int N> __device__ __forceinline__ LaneSum<C> &lane_of(LaneSum<C> (&a)[N], int u) { return a[u]; }
 
-// LAST: the group may reach past n.  Entries there are neither loaded nor
-// stored and add +0, which changes no sum (sums start from +0 and are never -0):
-// leaving the loop at the first of them instead put every add behind its own
-// branch (one-launch FAST update of 5000 entries 7.9 us against 5.0).
-template <int KIND, int U, bool NT, bool LAST = false, typename ACC>
-__device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t stride, ACC &acc, int64_t n = 0) {
+template <int KIND, int U, bool NT, typename ACC>
+__device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t stride, ACC &acc) {
+  double va[U], vb[U], vr[U], vx[U];
+  int64_t ix[KIND == RED_CGFULL ? U : 1];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = id + u * stride;
+    if constexpr (KIND == RED_CGFULL) {
+      ix[u] = x_index(A, i);
+      va[u] = ldv<NT>(A.a + ix[u]);
+      vx[u] = ldv<NT>(A.x + ix[u]);
+    } else {
+      va[u] = ldv<NT>(A.a + i);
+    }
+    if constexpr (KIND == RED_DOT || KIND == RED_CGFULL) vb[u] = ldv<NT>(A.b + i);
+    if constexpr (KIND == RED_CG || KIND == RED_CGFULL) vr[u] = ldv<NT>(A.r + i);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = id + u * stride;
+    double term;
+    if constexpr (KIND == RED_NORM) {
+      term = va[u] * va[u];
+    } else if constexpr (KIND == RED_DOT) {
+      term = va[u] * vb[u];
+    } else if constexpr (KIND == RED_CG) {
+      const double rr = vr[u] + A.alpha * va[u];
+      stv<NT>(A.r + i, rr);
+      term = rr * rr;
+    } else {
+      stv<NT>(A.x + ix[u], vx[u] + A.alpha * va[u]);
+      const double rr = vr[u] - A.alpha * vb[u];
+      stv<NT>(A.r + i, rr);
+      term = rr * rr;
+    }
+    lane_of(acc, u).add(term);
+  }
+}
+
+// The same where the group may reach past n.  Entries there are neither loaded
+// nor stored and add +0, which changes no sum (sums start from +0 and are never
+// -0): leaving the loop at the first of them instead put every add behind its
+// own branch (one-launch FAST update of 5000 entries 7.9 us against 5.6).  Apart from
+// ref_group, whose loads it would otherwise reorder (full form of 2^27
+// entries 1100 us against 1115).
+template <int KIND, int U, bool NT, typename ACC>
+__device__ __forceinline__ void ref_group_last(const RedArgs &A, int64_t id, int64_t stride, ACC &acc, int64_t n) {
   double va[U], vb[U], vr[U], vx[U];
   int64_t ix[KIND == RED_CGFULL ? U : 1];
 #pragma unroll
@@ -222,7 +263,7 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
     const int64_t i = id + u * stride;
     va[u] = vb[u] = vr[u] = vx[u] = 0.0;
     if constexpr (KIND == RED_CGFULL) ix[u] = x_index(A, i);
-    if (!LAST || i < n) {
+    if (i < n) {
       if constexpr (KIND == RED_CGFULL) {
         va[u] = ldv<NT>(A.a + ix[u]);
         vx[u] = ldv<NT>(A.x + ix[u]);
@@ -236,7 +277,6 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t i = id + u * stride;
-    const bool in = !LAST || i < n;
     double term;
     if constexpr (KIND == RED_NORM) {
       term = va[u] * va[u];
@@ -244,17 +284,17 @@ __device__ __forceinline__ void ref_group(const RedArgs &A, int64_t id, int64_t 
       term = va[u] * vb[u];
     } else if constexpr (KIND == RED_CG) {
       const double rr = vr[u] + A.alpha * va[u];
-      if (in) stv<NT>(A.r + i, rr);
+      if (i < n) stv<NT>(A.r + i, rr);
       term = rr * rr;
     } else {
       const double rr = vr[u] - A.alpha * vb[u];
-      if (in) {
+      if (i < n) {
         stv<NT>(A.x + ix[u], vx[u] + A.alpha * va[u]);
         stv<NT>(A.r + i, rr);
       }
       term = rr * rr;
     }
-    lane_of(acc, u).add(in ? term : 0.0);
+    lane_of(acc, u).add(i < n ? term : 0.0);
   }
 }
 
@@ -284,7 +324,7 @@ __global__ __launch_bounds__(BS) void k_red_ref1(int64_t n, int64_t nblock, RedA
       }
     }
     for (; id + 3 * stride < n; id += 4 * stride) ref_group<KIND, 4, NT>(A, id, stride, acc);
-    if (id < n) ref_group<KIND, 4, NT, true>(A, id, stride, acc, n);
+    if (id < n) ref_group_last<KIND, 4, NT>(A, id, stride, acc, n);
   } else {
     for (; id < n; id += stride) acc.add(red_term<KIND>(A, id));
   }
@@ -353,7 +393,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_red_small(int64_t n, int n
     LaneSum<COMP> acc[4 * G];
     const int64_t i0 = (int64_t)b * 256;
     if (i0 + 256 * G <= n) ref_group<KIND, 4 * G, false>(A, i0 + l, 64, acc);
-    else ref_group<KIND, 4 * G, false, true>(A, i0 + l, 64, acc, n);
+    else ref_group_last<KIND, 4 * G, false>(A, i0 + l, 64, acc, n);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const LaneSum<COMP> *e = acc + 4 * g;
