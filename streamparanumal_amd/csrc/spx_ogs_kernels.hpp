@@ -483,7 +483,10 @@ __device__ __forceinline__ void pack_rows(unsigned lead, Use &&use) {
 // positions (pack_rows), once for all rounds.  Measured, us per call, without /
 // with: FP32 values, K = 3, 48x47x46 p=4 83.6 / 79.0, a batch of 16 uneven
 // boxes with its CG update 378 / 369; small operators' tiles of 4 positions
-// per lane lose (FP32, K = 2, 172224-node Tri p=1 5.4 / 5.8).
+// per lane lose (FP32, K = 2, 172224-node Tri p=1 5.4 / 5.8).  Where rows are long
+// and few it gains little or loses a little: FP64 K = 2 44^3 p=7 234 / 238, K = 4 36^3 p=7
+// 430 / 444 (28^3 235 / 225, 44^3 798 / 798), FP32 sums K = 2 28^3 p=7 41.2 / 42.0 (36^3
+// 89.5 / 87.7), FP32 storage K = 2 10^3 p=15 17.4 / 17.8, 24^3 p=9 48.6 / 49.8.
 template <int KF, int PER> constexpr bool kPackRows = KF > 1 && PER >= 8;
 
 template <typename T, int OP, int KF, int PER, int NT = kThreads, typename F = Fold<T, OP>, int MODE = kAll,

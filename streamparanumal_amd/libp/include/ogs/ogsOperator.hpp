@@ -194,7 +194,9 @@ class ogsOperator_t {
   // unless the caller chose row blocks or a layout of them: their stores are whole 16-byte words
   // in order.  Row tiles / local order, us per call: FP64 one field 12^3 p=7
   // 7.0 / 5.2, 48^3 p=7 171 / 150, 64^3 p=7 384 / 361, 29^3 p=15 334 / 293,
-  // 1250^2 Quad p=7 291 / 279; FP32 64^3 p=7 286 / 231.  The N-CSR scatter of a
+  // 1250^2 Quad p=7 291 / 279; FP32 64^3 p=7 286 / 231.  (Where the setup picks
+  // local order anyway, a lane per node beat the words on one mesh of those tried, 400^2 Tri
+  // p=3: FP64 K = 2 14.2 / 14.5, K = 3 21.0 / 22.2, K = 4 26.9 / 28.4.)  The N-CSR scatter of a
   // Signed operator stores to single nodes, and more fields one at a time:
   // those keep the rule on row length.
   // So do unaligned vectors, but for those whose stores need no alignment
